@@ -92,6 +92,309 @@ __global__ __launch_bounds__(256) void append_kernel(const AppendArgs a) {
   store_token<DP, BITS>(g, head, slot, kc, vc, s_meta[wave][0], s_meta[wave][1], lane);
 }
 
+// ---- append of several tokens per sequence: one wave per 16-token tile side -----
+//
+// The row kernel above scatters a token's codes byte by byte into the tile
+// payloads (64 separate lines per V row) and spends a wave, and two row reads,
+// on every padding row of a ragged batch.  With several tokens per sequence
+// the unit here is one side (K or V) of a page tile of one (sequence, KV
+// head): lane (t, jj) holds the elements d = 32*kb + 8*jj + e of token t --
+// 16-byte loads, and, once quantized, exactly the lane's share of the K
+// payload (16-byte stores).  V is quantized the same way and turned to its
+// column order through LDS.  HBM-bound for long chunks: 16 sequences x 1,024
+// tokens x 8 heads x 128 to int8 (103 MB) 106 -> 25.5 us (4.0 TB/s), 4-bit
+// 101 -> 23 us, f16 pages 94 -> 29 us; 36 sequences padded to 512 tokens, 32
+// of them one token wide, 48 -> 15 us.
+// The division by the group's scale is one reciprocal per group and three
+// operations per element (Markstein: with y = RN(1/s) and q = RN(n*y),
+// RN(q + y*(n - q*s)) is the correctly rounded n/s), so codes are the row
+// kernel's bit for bit; a wave that meets infinities, NaN or a range past f16
+// (where that identity fails) does the row kernel's operations.
+
+// 8 float_kind elements in 16 bytes -> f32
+template <int FK>
+__device__ __forceinline__ void unpack8(const u4 &v, float (&x)[8]) {
+  const uint32_t w[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    x[2 * i] = bits_to_float((uint16_t)(w[i] & 0xFFFFu), FK);
+    x[2 * i + 1] = bits_to_float((uint16_t)(w[i] >> 16), FK);
+  }
+}
+
+// Quantize the lane's share of its token's row: meta words of every storage
+// group and the codes, 8 per kb, as two words of four bytes.  The whole wave
+// calls.
+template <int DP, int G, int BITS, int FK>
+__device__ __forceinline__ void quantize_share(const u4 (&raw)[DP / 32], uint32_t (&meta)[DP / G],
+                                               uint32_t (&codes)[DP / 16]) {
+  constexpr int NG = DP / G, KPG = G / 32;
+  const float levels = (float)((1 << BITS) - 1);
+  float lo[NG], hi[NG], bias[NG], scale[NG];
+  auto affine = [&](int gi) __attribute__((always_inline)) {
+    const uint16_t b16 = f32_to_f16_bits(lo[gi]);
+    bias[gi] = f16_bits_to_f32(b16);
+    const uint16_t s16 = f32_to_f16_bits(fmaxf(__fdiv_rn(hi[gi] - bias[gi], levels), 1e-6f));
+    scale[gi] = f16_bits_to_f32(s16);
+    meta[gi] = (uint32_t)s16 | ((uint32_t)b16 << 16);
+  };
+  // min and max by the NaN-propagating three-input forms (half the operations
+  // of fminf / fmaxf, and no canonicalisation)
+  bool odd = false;
+#pragma unroll
+  for (int gi = 0; gi < NG; ++gi) {
+    float l = 0.0f, h = 0.0f;
+#pragma unroll
+    for (int k = 0; k < KPG; ++k) {
+      float x[8];
+      unpack8<FK>(raw[gi * KPG + k], x);
+      if (k == 0) l = h = x[0];
+#pragma unroll
+      for (int e = 0; e < 8; e += 2) {
+        l = __builtin_elementwise_minimum(__builtin_elementwise_minimum(x[e], x[e + 1]), l);
+        h = __builtin_elementwise_maximum(__builtin_elementwise_maximum(x[e], x[e + 1]), h);
+      }
+    }
+    l = __builtin_elementwise_minimum(l, __shfl_xor(l, 16, 64));
+    h = __builtin_elementwise_maximum(h, __shfl_xor(h, 16, 64));
+    lo[gi] = __builtin_elementwise_minimum(l, __shfl_xor(l, 32, 64));
+    hi[gi] = __builtin_elementwise_maximum(h, __shfl_xor(h, 32, 64));
+    affine(gi);
+    odd |= !(fabsf(bias[gi]) < INFINITY && scale[gi] < INFINITY && hi[gi] - lo[gi] < INFINITY);
+  }
+  if (__any(odd)) {  // rare: infinities, NaN, or a range past f16: the row kernel's operations
+#pragma unroll
+    for (int gi = 0; gi < NG; ++gi) {
+      float l = 0.0f, h = 0.0f;
+#pragma unroll
+      for (int k = 0; k < KPG; ++k) {
+        float x[8];
+        unpack8<FK>(raw[gi * KPG + k], x);
+        if (k == 0) l = h = x[0];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) { l = fminf(l, x[e]); h = fmaxf(h, x[e]); }
+      }
+      lo[gi] = xor32_min(xor16_min(l));
+      hi[gi] = xor32_max(xor16_max(h));
+      affine(gi);
+    }
+#pragma unroll
+    for (int kb = 0; kb < DP / 32; ++kb) {
+      float x[8];
+      unpack8<FK>(raw[kb], x);
+      uint32_t w[2] = {0, 0};
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        float c = rintf(__fdiv_rn(x[e] - bias[kb / KPG], scale[kb / KPG]));
+        c = fminf(fmaxf(c, 0.0f), levels);
+        w[e / 4] |= (uint32_t)c << (8 * (e % 4));
+      }
+      codes[2 * kb] = w[0];
+      codes[2 * kb + 1] = w[1];
+    }
+    return;
+  }
+  float rcp[NG];
+#pragma unroll
+  for (int gi = 0; gi < NG; ++gi) rcp[gi] = __fdiv_rn(1.0f, scale[gi]);
+#pragma unroll
+  for (int kb = 0; kb < DP / 32; ++kb) {
+    const int gi = kb / KPG;
+    float x[8];
+    unpack8<FK>(raw[kb], x);
+    uint32_t c[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const float n = x[e] - bias[gi];
+      float q = n * rcp[gi];
+      q = __builtin_fmaf(__builtin_fmaf(-q, scale[gi], n), rcp[gi], q);
+      // clamped, then rounded half to even into the low bits of 1.5 * 2^23 + c
+      // (the bounds are integers: rounding first gives the same code)
+      c[e] = __float_as_uint(__builtin_amdgcn_fmed3f(q, 0.0f, levels) + 12582912.0f);
+    }
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const uint32_t p01 = __builtin_amdgcn_perm(c[4 * i + 1], c[4 * i], 0x0C0C0400u);
+      const uint32_t p23 = __builtin_amdgcn_perm(c[4 * i + 3], c[4 * i + 2], 0x04000C0Cu);
+      codes[2 * kb + i] = p01 | p23;
+    }
+  }
+}
+
+template <int DP, int G, int BITS>
+__global__ __launch_bounds__(256) void append_tiles_kernel(const AppendArgs a, int tiles, bool vec) {
+  constexpr int KB = DP / 32, NB = DP / 16;
+  constexpr int ROWW = BITS == 16 ? DP / 2 + 4 : DP / 4 + 4;  // V rows in LDS, words
+  __shared__ __attribute__((aligned(16))) uint32_t s_v[4][16 * ROWW];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const Geo &g = a.g;
+  const int64_t item = (int64_t)blockIdx.x * 4 + wave;
+  if (item >= (int64_t)a.batch * g.hk * tiles * 2) return;
+  // neighbouring waves take neighbouring tiles of one side
+  const int ti = (int)(item % tiles);
+  const int side = (int)((item / tiles) & 1);
+  const int kh = (int)((item / tiles / 2) % g.hk);
+  const int b = (int)(item / ((int64_t)tiles * 2 * g.hk));
+  const int width = min(a.widths ? a.widths[b] : a.tokens, a.tokens);
+  const int start = a.start_pos ? a.start_pos[b] : a.lens_after[b] - a.tokens;
+  if (a.new_lens && ti == 0 && kh == 0 && side == 0 && lane == 0)
+    a.new_lens[b] = start + (a.widths ? a.widths[b] : a.tokens);
+  // the ti-th tile the new positions [max(start, 0), start + width) touch
+  const int tile = max(start, 0) / PKV_TILE + ti;
+  const int pos0 = tile * PKV_TILE;
+  if (width <= 0 || pos0 >= start + width || pos0 / g.page >= a.max_pages) return;
+  const int page = a.table[(int64_t)b * a.max_pages + pos0 / g.page];  // read beside the rows
+  const int t = lane & 15, jj = lane >> 4;
+  const int tok = pos0 + t - start;  // the lane's token among the new ones
+  const bool mine = tok >= 0 && tok < width;
+  const int64_t row = (((int64_t)b * g.hk + kh) * a.tokens + (mine ? tok : 0)) * g.dim;
+  const uint16_t *src = (side ? a.values : a.keys) + row;
+  u4 raw[KB];
+#pragma unroll
+  for (int kb = 0; kb < KB; ++kb) {
+    const int d0 = 32 * kb + 8 * jj;
+    u4 v = {0, 0, 0, 0};  // zero pad past the head dim
+    if (vec) {
+      if (mine && d0 < g.dim) v = *(const u4 *)(src + d0);
+    } else if (mine) {
+      uint32_t e8[8];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) e8[e] = d0 + e < g.dim ? src[d0 + e] : (uint16_t)0;
+      v = u4{e8[0] | (e8[1] << 16), e8[2] | (e8[3] << 16), e8[4] | (e8[5] << 16), e8[6] | (e8[7] << 16)};
+    }
+    raw[kb] = v;
+  }
+  if (page < 0 || page >= a.num_pages) return;
+  uint8_t *head = a.pool + (int64_t)page * g.page_bytes + (int64_t)kh * g.head_bytes;
+  const int slot0 = pos0 % g.page;
+  const int64_t toff = (int64_t)(slot0 / PKV_TILE) * g.tile_bytes;
+  uint8_t *ktile = head + toff, *vtile = head + g.v_offset + toff;
+  uint32_t *vrow = s_v[wave] + t * ROWW;
+  if constexpr (BITS == 16) {
+    if (side == 0) {
+      if (mine) {
+#pragma unroll
+        for (int kb = 0; kb < KB; ++kb) *(u4 *)(ktile + kb * 1024 + lane * 16) = raw[kb];
+      }
+      return;
+    }
+#pragma unroll
+    for (int kb = 0; kb < KB; ++kb) *(u4 *)(vrow + 16 * kb + 4 * jj) = raw[kb];
+  } else {
+    constexpr int NG = DP / G;
+    uint32_t meta[NG], codes[2 * KB];
+    if (g.float_kind == 0) quantize_share<DP, G, BITS, 0>(raw, meta, codes);
+    else quantize_share<DP, G, BITS, 1>(raw, meta, codes);
+    if (mine) {
+      // the token's (scale, bias) words: group gi by lane jj = gi % 4
+      uint32_t *m = (uint32_t *)(head + (side ? g.vmeta_offset : g.kmeta_offset)) + (slot0 + t) * NG;
+#pragma unroll
+      for (int gi = 0; gi < NG; ++gi)
+        if (gi % 4 == jj) m[gi] = meta[gi];
+    }
+    if (side == 0) {
+      // K: the lane's payload, 16-byte chunks (8 bytes where it holds no more)
+      constexpr int LW = DP * BITS / 128;
+      uint32_t w[LW];
+#pragma unroll
+      for (int i = 0; i < LW; ++i) {
+        if constexpr (BITS == 8) {
+          w[i] = codes[i];
+        } else {
+          // nibble (e odd ? 4 : 0) + e / 2 holds element e
+          const uint32_t c0 = codes[2 * i], c1 = codes[2 * i + 1];
+          const uint32_t ev = (c0 & 15u) | ((c0 >> 12) & 0xF0u) | ((c1 & 15u) << 8) | ((c1 >> 4) & 0xF000u);
+          const uint32_t od = ((c0 >> 8) & 15u) | ((c0 >> 20) & 0xF0u) | (c1 & 0xF00u) | ((c1 >> 12) & 0xF000u);
+          w[i] = ev | (od << 16);
+        }
+      }
+      if (mine) {
+        if constexpr (LW >= 4) {
+#pragma unroll
+          for (int c = 0; c < LW / 4; ++c)
+            *(u4 *)(ktile + c * 1024 + lane * 16) = u4{w[4 * c], w[4 * c + 1], w[4 * c + 2], w[4 * c + 3]};
+        } else {
+          *(u2 *)(ktile + lane * 8) = u2{w[0], w[1]};
+        }
+      }
+      return;
+    }
+    // codes of d = 32*kb + 8*jj + 0..7: words 8*kb + 2*jj, + 1 of the row
+#pragma unroll
+    for (int kb = 0; kb < KB; ++kb) *(u2 *)(vrow + 8 * kb + 2 * jj) = u2{codes[2 * kb], codes[2 * kb + 1]};
+  }
+  wave_lds_sync();
+  // V: lane (col, jj) takes column d = 16*n + col of tokens 4*jj .. 4*jj + 3
+  const int col = t;
+  const int first = pos0 + 4 * jj - start;  // token 4*jj of the tile, among the new ones
+  const bool all4 = first >= 0 && first + 3 < width;
+  const uint32_t *vcol = s_v[wave] + 4 * jj * ROWW;
+  if constexpr (BITS == 16) {
+    const uint32_t sel = (col & 1) ? 0x07060302u : 0x05040100u;
+    uint32_t w[2 * NB];
+#pragma unroll
+    for (int n = 0; n < NB; ++n) {
+      uint32_t r[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) r[i] = vcol[i * ROWW + 8 * n + (col >> 1)];
+      w[2 * n] = __builtin_amdgcn_perm(r[1], r[0], sel);
+      w[2 * n + 1] = __builtin_amdgcn_perm(r[3], r[2], sel);
+    }
+    if (all4) {
+#pragma unroll
+      for (int c = 0; c < NB / 2; ++c)
+        *(u4 *)(vtile + c * 1024 + lane * 16) = u4{w[4 * c], w[4 * c + 1], w[4 * c + 2], w[4 * c + 3]};
+    } else {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        if (first + i < 0 || first + i >= width) continue;
+#pragma unroll
+        for (int n = 0; n < NB; ++n)
+          *(uint16_t *)(vtile + (n / 2) * 1024 + lane * 16 + 8 * (n & 1) + 2 * i) =
+              (uint16_t)(w[2 * n + i / 2] >> (16 * (i & 1)));
+      }
+    }
+  } else {
+    // a word's bytes: tokens 0..3 of a column (8-bit), or 0, 2, 1, 3 with the
+    // odd block's codes in the high nibbles (4-bit)
+    const uint32_t cb = col & 3;
+    const uint32_t sel = cb | ((4 + cb) << 8) | 0x0C0C0000u;  // bytes cb of both sources
+    uint32_t w[NB];
+#pragma unroll
+    for (int n = 0; n < NB; ++n) {
+      uint32_t r[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) r[i] = vcol[i * ROWW + 4 * n + (col >> 2)];
+      const uint32_t p01 = __builtin_amdgcn_perm(r[BITS == 8 ? 1 : 2], r[0], sel);
+      const uint32_t p23 = __builtin_amdgcn_perm(r[3], r[BITS == 8 ? 2 : 1], sel);
+      w[n] = p01 | (p23 << 16);
+    }
+    constexpr int LW = DP * BITS / 128;
+    uint32_t o[LW];
+#pragma unroll
+    for (int i = 0; i < LW; ++i) o[i] = BITS == 8 ? w[i] : w[2 * i] | (w[2 * i + 1] << 4);
+    if (all4) {
+      if constexpr (LW >= 4) {
+#pragma unroll
+        for (int c = 0; c < LW / 4; ++c)
+          *(u4 *)(vtile + c * 1024 + lane * 16) = u4{o[4 * c], o[4 * c + 1], o[4 * c + 2], o[4 * c + 3]};
+      } else {
+        *(u2 *)(vtile + lane * 8) = u2{o[0], o[1]};
+      }
+    } else {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        if (first + i < 0 || first + i >= width) continue;
+        const int byte = BITS == 8 ? i : v4_byte(i);
+#pragma unroll
+        for (int x = 0; x < LW; ++x)
+          vtile[payload_offset(lane, 4 * x + byte, LW >= 4 ? 16 : 8)] = (uint8_t)(o[x] >> (8 * byte));
+      }
+    }
+  }
+}
+
 // ---- gather to the reference format ---------------------------------------
 
 
@@ -181,6 +484,32 @@ __global__ __launch_bounds__(256) void copy_pages_kernel(uint8_t *pool, int64_t 
 hipError_t launch_append(hipStream_t stream, const AppendArgs &a) {
   const int64_t items = (int64_t)a.batch * a.tokens * a.g.hk;
   if (items == 0) return hipSuccess;
+  // Tiles past half a tile of new tokens: below, a wave's 32 elements per lane
+  // are a longer chain than the row kernel's two (a 5-token verify step of 16
+  // sequences: 32.4 us by rows, 33.7 by tiles; 16 x 12 tokens alone: 4.5 us by
+  // rows, 3.8 by tiles).
+  if (a.tokens > PKV_TILE / 2) {
+    // tiles the new tokens of one sequence can touch (the first may be begun)
+    const int tiles = (a.tokens + 2 * PKV_TILE - 2) / PKV_TILE;
+    const int64_t blocks = ((int64_t)a.batch * a.g.hk * tiles * 2 + 3) / 4;
+    if (blocks > 0x7FFFFFFF) return hipErrorInvalidValue;
+    // 16-byte row loads need rows and tensors at 16-byte addresses
+    const bool vec = a.g.dim % 8 == 0 && ((uintptr_t)a.keys & 15) == 0 && ((uintptr_t)a.values & 15) == 0;
+    dim3 grid((unsigned)blocks), block(256);
+#define PKV_TILES(DP_, G_, BITS_)                                                                     \
+  if (a.g.dp == DP_ && a.g.bits == BITS_ && (BITS_ == 16 || a.g.group == G_)) {                       \
+    hipLaunchKernelGGL((append_tiles_kernel<DP_, G_, BITS_>), grid, block, 0, stream, a, tiles, vec); \
+    return hipGetLastError();                                                                         \
+  }
+#define PKV_TILES_Q(DP_, G_) PKV_TILES(DP_, G_, 4) PKV_TILES(DP_, G_, 8)
+    PKV_TILES(64, 32, 16) PKV_TILES(128, 32, 16) PKV_TILES(256, 32, 16)
+    PKV_TILES_Q(64, 32) PKV_TILES_Q(64, 64)
+    PKV_TILES_Q(128, 32) PKV_TILES_Q(128, 64) PKV_TILES_Q(128, 128)
+    PKV_TILES_Q(256, 32) PKV_TILES_Q(256, 64) PKV_TILES_Q(256, 128)
+#undef PKV_TILES_Q
+#undef PKV_TILES
+    return hipErrorInvalidValue;
+  }
   dim3 grid((unsigned)((items + 3) / 4)), block(256);
 #define PKV_APPEND(DP_, BITS_)                                                       \
   if (a.g.dp == DP_ && a.g.bits == BITS_) {                                          \

@@ -108,6 +108,14 @@ __device__ __forceinline__ float xor32_add(float v) {
   const auto z = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
   return __uint_as_float(z[0]) + __uint_as_float(z[1]);
 }
+__device__ __forceinline__ float xor16_min(float v) {
+  const auto z = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return fminf(__uint_as_float(z[0]), __uint_as_float(z[1]));
+}
+__device__ __forceinline__ float xor32_min(float v) {
+  const auto z = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return fminf(__uint_as_float(z[0]), __uint_as_float(z[1]));
+}
 __device__ __forceinline__ float xor16_max(float v) {
   const auto z = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
   return fmaxf(__uint_as_float(z[0]), __uint_as_float(z[1]));
