@@ -104,23 +104,9 @@ __global__ __launch_bounds__(256) void append_kernel(const AppendArgs a) {
 // column order through LDS.  HBM-bound for long chunks: 16 sequences x 1,024
 // tokens x 8 heads x 128 to int8 (103 MB) 106 -> 25.5 us (4.0 TB/s), 4-bit
 // 101 -> 23 us, f16 pages 94 -> 29 us; 36 sequences padded to 512 tokens, 32
-// of them one token wide, 48 -> 15 us.
-// The division by the group's scale is one reciprocal per group and three
-// operations per element (Markstein: with y = RN(1/s) and q = RN(n*y),
-// RN(q + y*(n - q*s)) is the correctly rounded n/s), so codes are the row
-// kernel's bit for bit; a wave that meets infinities, NaN or a range past f16
-// (where that identity fails) does the row kernel's operations.
-
-// 8 float_kind elements in 16 bytes -> f32
-template <int FK>
-__device__ __forceinline__ void unpack8(const u4 &v, float (&x)[8]) {
-  const uint32_t w[4] = {v.x, v.y, v.z, v.w};
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    x[2 * i] = bits_to_float((uint16_t)(w[i] & 0xFFFFu), FK);
-    x[2 * i + 1] = bits_to_float((uint16_t)(w[i] >> 16), FK);
-  }
-}
+// of them one token wide, 48 -> 12.6 us.
+// The codes are the row kernel's bit for bit (codes8, pkv_token.h); a wave that
+// meets infinities, NaN or a range past f16 does the row kernel's operations.
 
 // Quantize the lane's share of its token's row: meta words of every storage
 // group and the codes, 8 per kb, as two words of four bytes.  The whole wave
@@ -149,11 +135,7 @@ __device__ __forceinline__ void quantize_share(const u4 (&raw)[DP / 32], uint32_
       float x[8];
       unpack8<FK>(raw[gi * KPG + k], x);
       if (k == 0) l = h = x[0];
-#pragma unroll
-      for (int e = 0; e < 8; e += 2) {
-        l = __builtin_elementwise_minimum(__builtin_elementwise_minimum(x[e], x[e + 1]), l);
-        h = __builtin_elementwise_maximum(__builtin_elementwise_maximum(x[e], x[e + 1]), h);
-      }
+      minmax8(x, l, h);
     }
     l = __builtin_elementwise_minimum(l, __shfl_xor(l, 16, 64));
     h = __builtin_elementwise_maximum(h, __shfl_xor(h, 16, 64));
@@ -182,15 +164,7 @@ __device__ __forceinline__ void quantize_share(const u4 (&raw)[DP / 32], uint32_
     for (int kb = 0; kb < DP / 32; ++kb) {
       float x[8];
       unpack8<FK>(raw[kb], x);
-      uint32_t w[2] = {0, 0};
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        float c = rintf(__fdiv_rn(x[e] - bias[kb / KPG], scale[kb / KPG]));
-        c = fminf(fmaxf(c, 0.0f), levels);
-        w[e / 4] |= (uint32_t)c << (8 * (e % 4));
-      }
-      codes[2 * kb] = w[0];
-      codes[2 * kb + 1] = w[1];
+      codes8_div(x, bias[kb / KPG], scale[kb / KPG], levels, codes[2 * kb], codes[2 * kb + 1]);
     }
     return;
   }
@@ -202,22 +176,7 @@ __device__ __forceinline__ void quantize_share(const u4 (&raw)[DP / 32], uint32_
     const int gi = kb / KPG;
     float x[8];
     unpack8<FK>(raw[kb], x);
-    uint32_t c[8];
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      const float n = x[e] - bias[gi];
-      float q = n * rcp[gi];
-      q = __builtin_fmaf(__builtin_fmaf(-q, scale[gi], n), rcp[gi], q);
-      // clamped, then rounded half to even into the low bits of 1.5 * 2^23 + c
-      // (the bounds are integers: rounding first gives the same code)
-      c[e] = __float_as_uint(__builtin_amdgcn_fmed3f(q, 0.0f, levels) + 12582912.0f);
-    }
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      const uint32_t p01 = __builtin_amdgcn_perm(c[4 * i + 1], c[4 * i], 0x0C0C0400u);
-      const uint32_t p23 = __builtin_amdgcn_perm(c[4 * i + 3], c[4 * i + 2], 0x04000C0Cu);
-      codes[2 * kb + i] = p01 | p23;
-    }
+    codes8(x, bias[gi], scale[gi], rcp[gi], levels, codes[2 * kb], codes[2 * kb + 1]);
   }
 }
 

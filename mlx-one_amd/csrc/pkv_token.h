@@ -43,6 +43,62 @@ __device__ __forceinline__ void quantize_row(const float (&x)[EPL], int lane, in
   if ((lane * EPL) % group == 0) meta[(lane * EPL) / group] = (uint32_t)s16 | ((uint32_t)b16 << 16);
 }
 
+// 8 float_kind elements in 16 bytes -> f32
+template <int FK>
+__device__ __forceinline__ void unpack8(const u4 &v, float (&x)[8]) {
+  const uint32_t w[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    x[2 * i] = bits_to_float((uint16_t)(w[i] & 0xFFFFu), FK);
+    x[2 * i + 1] = bits_to_float((uint16_t)(w[i] >> 16), FK);
+  }
+}
+
+// Running min and max with 8 more values, by the NaN-propagating three-input
+// forms (half the operations of fminf / fmaxf, and no canonicalisation).
+__device__ __forceinline__ void minmax8(const float (&x)[8], float &lo, float &hi) {
+#pragma unroll
+  for (int e = 0; e < 8; e += 2) {
+    lo = __builtin_elementwise_minimum(__builtin_elementwise_minimum(x[e], x[e + 1]), lo);
+    hi = __builtin_elementwise_maximum(__builtin_elementwise_maximum(x[e], x[e + 1]), hi);
+  }
+}
+
+// Codes of 8 elements of one group, one byte each, as the division by the
+// scale gives them.
+__device__ __forceinline__ void codes8_div(const float (&x)[8], float bias, float scale, float levels,
+                                           uint32_t &w0, uint32_t &w1) {
+  uint32_t w[2] = {0, 0};
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    float c = rintf(__fdiv_rn(x[e] - bias, scale));
+    c = fminf(fmaxf(c, 0.0f), levels);
+    w[e / 4] |= (uint32_t)c << (8 * (e % 4));
+  }
+  w0 = w[0];
+  w1 = w[1];
+}
+
+// The same codes where bias, scale and every x are finite, with rcp = 1 / scale
+// (rounded once): the correctly rounded quotient takes three operations per
+// element (Markstein: with y = RN(1/s) and q = RN(n*y), RN(q + y*(n - q*s)) is
+// RN(n/s)).
+__device__ __forceinline__ void codes8(const float (&x)[8], float bias, float scale, float rcp, float levels,
+                                       uint32_t &w0, uint32_t &w1) {
+  uint32_t c[8];
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    const float n = x[e] - bias;
+    float q = n * rcp;
+    q = __builtin_fmaf(__builtin_fmaf(-q, scale, n), rcp, q);
+    // clamped, then rounded half to even into the low bits of 1.5 * 2^23 + c
+    // (the bounds are integers: rounding first gives the same code)
+    c[e] = __float_as_uint(__builtin_amdgcn_fmed3f(q, 0.0f, levels) + 12582912.0f);
+  }
+  w0 = __builtin_amdgcn_perm(c[1], c[0], 0x0C0C0400u) | __builtin_amdgcn_perm(c[3], c[2], 0x04000C0Cu);
+  w1 = __builtin_amdgcn_perm(c[5], c[4], 0x0C0C0400u) | __builtin_amdgcn_perm(c[7], c[6], 0x04000C0Cu);
+}
+
 // Make one wave's LDS writes visible to its other lanes.
 __device__ __forceinline__ void wave_lds_sync() {
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
