@@ -101,7 +101,9 @@ int pkv_append_quantize(void *stream, const pkv_layout *layout, void *pool, int6
  * span several runs is merged by log-sum-exp (:191-204) in a second kernel on
  * the same stream.  Wider query
  * blocks (up to 2^24 rows per KV head) run on an MFMA prefill kernel, 256
- * rows per workgroup (128 at head_dim > 128), that needs no workspace.
+ * rows per workgroup (64 at head_dim > 128), that needs no workspace (with
+ * pkv_attention_batch_workspace_bytes of it, spans are cut into pieces where
+ * the row blocks are too few to fill the device).
  * Mixed batches (the reference pads decode and prefill rows into one call,
  * engine/paged.py:345-346, :384-389): in a wide call with `widths`, the
  * sequences whose width fits the decode kernel (at most 32 / (H/HK) queries,
@@ -223,6 +225,17 @@ int32_t pkv_attention_default_waves(const pkv_layout *layout, int32_t num_heads,
  * decode part (0 when the GQA ratio leaves the decode kernel no query). */
 int64_t pkv_attention_workspace_bytes(const pkv_layout *layout, int32_t num_heads,
                                       int32_t num_queries, int32_t waves);
+
+/* Workspace bytes with which pkv_paged_attention also runs a wide call
+ * (query blocks served by the prefill kernel) of `batch` sequences best: the
+ * partials of its decode parts side by side (merged in one launch) and those of
+ * prefill spans cut into pieces where the row blocks would leave compute units
+ * idle (f32, merged by the same launch).  At least
+ * pkv_attention_workspace_bytes(...), and equal to it for calls the decode
+ * kernel serves whole; a wide call accepts any smaller workspace, as before,
+ * and then cuts no span.  <0 on error. */
+int64_t pkv_attention_batch_workspace_bytes(const pkv_layout *layout, int32_t num_heads,
+                                            int32_t num_queries, int32_t batch, int32_t waves);
 
 /*
  * Copy pages out of the pool into the reference's per-page tensor format

@@ -77,6 +77,31 @@ WorkspaceParts workspace_parts(const pkv_geometry &g, int64_t rows, int64_t wave
   return w;
 }
 
+// Partials of split prefill spans (prefill_split) for a wide call of `batch`
+// sequences: [pieces per row block: int32][ml][acc] with `blocks` pieces of one
+// workgroup's rows each; no blocks where no span can be split.  `share`: a
+// mixed batch, whose live sequences the host does not know (one or more).
+struct PrefillParts {
+  int cus;  // 0: no split
+  int64_t blocks, ml, acc, total;
+};
+
+PrefillParts prefill_parts(const pkv_geometry &g, int64_t rows, int64_t batch, bool share) {
+  PrefillParts p{0, 0, 0, 0, 0};
+  const pkv::Geo geo = pkv::to_geo(g);
+  const int cus = pkv::device_cus();
+  const int64_t per_seq = (int64_t)g.hk * pkv::prefill_blocks(geo, (int)rows);
+  const int64_t least = share ? per_seq : per_seq * batch;
+  if (cus <= 0 || pkv::prefill_split(least, cus) < 2) return p;
+  p.cus = cus;
+  p.blocks = share ? 2 * (int64_t)cus : least * pkv::prefill_split(least, cus);
+  const int64_t block_rows = pkv::prefill_block_rows(geo);
+  p.ml = align256(p.blocks * 4);
+  p.acc = p.ml + align256(p.blocks * block_rows * 2 * 4);
+  p.total = p.acc + align256(p.blocks * block_rows * g.dp * 4);
+  return p;
+}
+
 // Resident-wave capacity per (device, layout, rows), measured once.
 int cached_waves(const pkv_geometry &geo, int rows) {
   static std::mutex mu;
@@ -213,6 +238,24 @@ int64_t pkv_attention_workspace_bytes(const pkv_layout *layout, int32_t num_head
   return workspace_parts(g, rows, waves).total;
 }
 
+int64_t pkv_attention_batch_workspace_bytes(const pkv_layout *layout, int32_t num_heads, int32_t num_queries,
+                                            int32_t batch, int32_t waves) {
+  const int64_t need = pkv_attention_workspace_bytes(layout, num_heads, num_queries, waves);
+  pkv_geometry g;
+  if (need < 0 || batch < 1 || geometry(layout, &g) != PKV_OK) return need < 0 ? need : -1;
+  const int gqa = num_heads / g.hk;
+  const int64_t rows = (int64_t)num_queries * gqa;
+  if (pkv::decode_serves(pkv::to_geo(g), (int)rows)) return need;
+  // a wide call: every decode part's partials side by side, and the split spans'
+  const int hi = decode_queries(g, gqa);
+  const int lo = std::min(hi, 4 / std::max(gqa, 1));
+  int64_t parts = 0;
+  if (lo >= 1) parts += align256(workspace_parts(g, (int64_t)lo * gqa, waves, 0).total);
+  if (hi > lo) parts += align256(workspace_parts(g, (int64_t)hi * gqa, waves, 0).total);
+  const int64_t mixed = parts + prefill_parts(g, rows, batch, hi >= 1).total;
+  return std::max(need, std::max(mixed, prefill_parts(g, rows, batch, false).total));
+}
+
 }  // extern "C"
 
 namespace {
@@ -303,6 +346,28 @@ int paged_attention_impl(void *stream, const pkv_layout *layout, const void *poo
     }
   }
 
+  // A wide call with room for them all keeps each part's partials in a region of
+  // its own, so that one launch merges them, and cuts prefill spans into pieces
+  // where its row blocks leave CUs idle.  (A workspace sized for the decode parts
+  // alone, and the library's own scratch, run the parts and their merges one
+  // after the other over one region, and no span is cut.)
+  PrefillParts pre{0, 0, 0, 0, 0};
+  bool together = false;
+  int64_t part_base[2] = {0, 0};
+  if (wide && !fit_waves && workspace) {
+    pre = prefill_parts(geo, rows, batch, nparts > 0);
+    int64_t total = pre.total;
+    for (int i = 0; i < nparts; ++i) {
+      part_base[i] = total;
+      total += align256(part[i].ws.total);
+    }
+    together = workspace_bytes >= total && total > 0;
+    if (!together) {
+      pre = PrefillParts{0, 0, 0, 0, 0};
+      part_base[0] = part_base[1] = 0;
+    }
+  }
+
   // The fused append: in the decode kernel when it serves the shape, else
   // one append launch ahead of the attention.
   if (fused) {
@@ -355,8 +420,16 @@ int paged_attention_impl(void *stream, const pkv_layout *layout, const void *poo
     a.lead = 0;
     a.part_ml = nullptr;
     a.part_acc = nullptr;
+    if (pre.cus > 0) {
+      a.pre_cus = pre.cus;
+      a.pre_cnt = (int32_t *)workspace;
+      a.pre_ml = (float *)((char *)workspace + pre.ml);
+      a.pre_acc = (float *)((char *)workspace + pre.acc);
+    }
     if (int rc = check_launch(pkv::launch_prefill((hipStream_t)stream, a), "prefill launch")) return rc;
   }
+  const pkv::AttnArgs wide_args = a;
+  pkv::MergeArgs merges[2];
   for (int i = 0; i < nparts; ++i) {
     const Part &t = part[i];
     a.nq = t.nq;
@@ -365,8 +438,8 @@ int paged_attention_impl(void *stream, const pkv_layout *layout, const void *poo
     a.narrow_q = t.hi;
     a.waves = (int)attention_runs(geo, a.rows, t.waves, fused != nullptr);
     a.lead = pkv::attention_lead(a.g, a.rows, fused != nullptr);
-    a.part_ml = (float *)((char *)workspace + t.ws.ml);
-    a.part_acc = (float *)((char *)workspace + t.ws.acc);
+    a.part_ml = (float *)((char *)workspace + part_base[i] + t.ws.ml);
+    a.part_acc = (float *)((char *)workspace + part_base[i] + t.ws.acc);
     if (fused) {
       a.wpool = (uint8_t *)fused->pool;
       a.new_k = (const uint16_t *)fused->keys;
@@ -374,7 +447,7 @@ int paged_attention_impl(void *stream, const pkv_layout *layout, const void *poo
     }
     if (int rc = check_launch(pkv::launch_attention((hipStream_t)stream, a), "attention launch"))
       return rc;
-    pkv::MergeArgs m;
+    pkv::MergeArgs &m = merges[i];
     m.batch = batch;
     m.hk = geo.hk;
     m.heads = num_heads;
@@ -394,8 +467,12 @@ int paged_attention_impl(void *stream, const pkv_layout *layout, const void *poo
     m.part_acc = a.part_acc;
     m.part_ml = a.part_ml;
     m.out = (uint16_t *)out;
+    if (together) continue;
     if (int rc = check_launch(pkv::launch_merge((hipStream_t)stream, m), "merge launch")) return rc;
   }
+  if (together)
+    return check_launch(pkv::launch_tail_merge((hipStream_t)stream, merges, nparts, wide_args, pre.cus > 0),
+                        "merge launch");
   return PKV_OK;
 }
 

@@ -51,6 +51,7 @@
 #include <atomic>
 #include <type_traits>
 
+#include "pkv_merge.h"
 #include "pkv_mfma.h"
 #include "pkv_token.h"
 
@@ -90,233 +91,9 @@ constexpr bool kDequantRows = true;
 // append) run one wave per run.
 constexpr int run_waves(int rb, int slots, bool append) { return !append && (rb == 2 || slots == 2) ? 4 : 1; }
 
-// Tiles of a sequence: at least one, so that an empty sequence still owns a
-// piece that writes its zero output.
-__device__ __forceinline__ int seq_tiles(int len) {
-  return len <= 0 ? 1 : (len + PKV_TILE - 1) / PKV_TILE;
-}
-
-// Work split.  Split tiles are numbered over (sequence b, KV head kh) in that
-// order, T in all: each (b, kh) segment spans `lead` tiles with no data, then
-// its own tiles.  Wave w of W (W <= T) owns the run [start(w), start(w+1)):
-// equal runs whatever the lengths, so no wave waits on a ragged tail and each
-// pays its start-up once.  A run is cut into pieces at segment boundaries; a
-// run that holds lead tiles only has no piece.
-struct Split {
-  int T, W, q, r;  // T tiles over W waves: the first r runs have q + 1 tiles, the rest q
-  __device__ __forceinline__ void init(int t, int w) {
-    T = t; W = w; q = t / w; r = t - q * w;
-  }
-  __device__ __forceinline__ int start(int w) const { return w * q + min(w, r); }
-  // the wave whose run holds tile g
-  __device__ __forceinline__ int wave_of(int g) const {
-    const int big = r * (q + 1);
-    return g < big ? g / (q + 1) : r + (g - big) / q;
-  }
-};
-
-// Partial slots: the first piece of wave w's run goes to slot 2w, a later
-// (its last) one to 2w+1; pieces in between cover whole segments and write
-// the output directly.  A segment starting at split tile sv has its tiles at
-// [s0, s1) (s0 = sv + lead); its pieces are those of waves wa .. wa+n-1, and
-// wave wa's piece is its first one unless its run started before sv.
-struct SegPieces {
-  int n, wa, slot0;
-  __device__ __forceinline__ int slot(int i) const { return i == 0 ? slot0 : 2 * (wa + i); }
-};
-
-__device__ __forceinline__ SegPieces seg_pieces(const Split &sp, int sv, int s0, int s1) {
-  SegPieces p;
-  p.wa = sp.wave_of(s0);
-  p.n = sp.wave_of(s1 - 1) - p.wa + 1;
-  p.slot0 = sp.start(p.wa) < sv ? 2 * p.wa + 1 : 2 * p.wa;
-  return p;
-}
-
-// Tiles the split gives sequence idx (< batch): seq_tiles, or none for a
-// sequence of a mixed batch that the prefill kernel serves (its width is past
-// narrow_q, the query rows this launch covers).  Served sequences have at
-// least one tile, so "served" is "tiles > 0", and only they are charged lead
-// tiles.
-__device__ __forceinline__ int split_tiles(const int32_t *lens, const int32_t *widths, int narrow_lo,
-                                           int narrow_q, int idx) {
-  if (narrow_q > 0 && (widths[idx] > narrow_q || widths[idx] <= narrow_lo)) return 0;
-  return seq_tiles(lens[idx]);
-}
-
-// The lead tiles a launch's split charges ahead of each segment: `lead`, or
-// none when the lead-free split's equal runs already end on segment
-// boundaries (every sequence's tile count a multiple of the run length), so
-// that no run crosses one.  nt0: the lane's tile count in the first
-// 64-sequence chunk; t0: the lead-free tile total over all segments.
-__device__ __forceinline__ int charged_lead(const int32_t *lens, const int32_t *widths, int narrow_lo,
-                                            int narrow_q, int batch, int waves, int lead, int nt0,
-                                            int t0, int lane) {
-  if (lead == 0 || t0 == 0) return 0;
-  const int w0 = min(waves, t0);
-  if (t0 % w0) return lead;
-  const int q0 = t0 / w0;
-  bool off = lane < batch && nt0 % q0 != 0;
-  for (int c0 = 64; c0 < batch; c0 += 64) {
-    const int idx = c0 + lane;
-    off |= idx < batch && split_tiles(lens, widths, narrow_lo, narrow_q, idx) % q0 != 0;
-  }
-  return __any(off) ? lead : 0;
-}
-
-// Log-sum-exp merge of partition partials (paged_attention.py:191-204, in
-// the exp2 domain): one NW-wave workgroup (1, 2 or 4 waves, as many as a
-// segment's pieces need at 16 per wave) per (segment, query
-// row) of a segment split over several waves' runs; whole segments were
-// written by the attention kernel.  Every wave finds M = max m and
-// S = sum l 2^(m - M) over the pieces (lanes stride the pieces); wave w
-// weighs pieces w, w+NW, ..., whose partial rows (lanes stride the DP
-// columns, up to 16 in flight) it requests before that pass, and the NW sums
-// meet in LDS.  Up to 16*NW pieces the merge is one memory round trip.
 template <int DP, int NW>
 __global__ __launch_bounds__(64 * NW) void merge_kernel(const MergeArgs a) {
-  constexpr int PER = DP / 64 > 0 ? DP / 64 : 1;  // output columns per lane
-  constexpr int KW = 16;                          // pieces per wave in flight
-  __shared__ float s_acc[NW > 1 ? NW - 1 : 1][64 * PER];
-  const int lane = threadIdx.x & 63;
-  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int unit = blockIdx.x;
-  const int row = unit % a.rows, seg = unit / a.rows;
-  const int b = seg / a.hk, kh = seg % a.hk;
-  // tiles (and served sequences) before sequence b, and the launch's split
-  // (as the attention kernel made it)
-  int pre = 0, spre = 0, tiles = 0, served = 0, nt0 = 0;
-  for (int c0 = 0; c0 < a.batch; c0 += 64) {
-    const int idx = c0 + lane;
-    const int nt = idx < a.batch ? split_tiles(a.seq_lens, a.widths, a.narrow_lo, a.narrow_q, idx) : 0;
-    if (c0 == 0) nt0 = nt;
-    tiles += wave_sum(nt);
-    served += wave_sum(nt > 0 ? 1 : 0);
-    pre += wave_sum(idx < b ? nt : 0);
-    spre += wave_sum(idx < b && nt > 0 ? 1 : 0);
-  }
-  const int ntb = split_tiles(a.seq_lens, a.widths, a.narrow_lo, a.narrow_q, b);
-  if (ntb == 0) return;  // served by the prefill kernel
-  const int t0 = __builtin_amdgcn_readfirstlane(tiles) * a.hk;
-  const int lead = charged_lead(a.seq_lens, a.widths, a.narrow_lo, a.narrow_q, a.batch, a.waves, a.lead, nt0,
-                                t0, lane);
-  const int T = t0 + __builtin_amdgcn_readfirstlane(served) * a.hk * lead;
-  const int sv = (__builtin_amdgcn_readfirstlane(pre) + __builtin_amdgcn_readfirstlane(spre) * lead) *
-                     a.hk + kh * (ntb + lead);
-  Split sp;
-  sp.init(T, min(a.waves, T));
-  const SegPieces pc = seg_pieces(sp, sv, sv + lead, sv + lead + ntb);
-  if (pc.n < 2) return;  // the same for every wave of the workgroup
-
-  // this wave's partial rows of pieces k0 + wv + NW*i, all requested at once
-  float x[KW][PER];
-  auto request = [&](int k0) __attribute__((always_inline)) {
-#pragma unroll
-    for (int i = 0; i < KW; ++i) {
-      const int k = k0 + wv + NW * i;
-#pragma unroll
-      for (int e = 0; e < PER; ++e) x[i][e] = 0.0f;
-      if (k < pc.n) {
-        const float *src = a.part_acc + ((int64_t)pc.slot(k) * a.rows + row) * DP + lane * PER;
-        if constexpr (PER == 4) {
-          const f4 v = *(const f4 *)src;
-          x[i][0] = v[0]; x[i][1] = v[1]; x[i][2] = v[2]; x[i][3] = v[3];
-        } else if constexpr (PER == 2) {
-          const float2 v = *(const float2 *)src;
-          x[i][0] = v.x; x[i][1] = v.y;
-        } else {
-          x[i][0] = src[0];
-        }
-      }
-    }
-  };
-  // The first rows go out before the (m, l) pass: both in one memory round trip.
-  request(0);
-
-  // M = max m, S = sum l 2^(m - M) over the pieces (lanes stride the pieces);
-  // lane l keeps piece l's (m, l)
-  float mx = -INFINITY, sm = 0.0f;
-  float2 mine = make_float2(-INFINITY, 0.0f);
-  for (int k0 = 0; k0 < pc.n; k0 += 64) {
-    const int k = k0 + lane;
-    if (k < pc.n) {
-      const float2 ml = *(const float2 *)(a.part_ml + ((int64_t)pc.slot(k) * a.rows + row) * 2);
-      if (k0 == 0) mine = ml;
-      if (ml.y > 0.0f) {  // a piece with no visible token holds l = 0
-        const float nm = fmaxf(mx, ml.x);
-        sm = sm * __builtin_amdgcn_exp2f(mx - nm) + ml.y * __builtin_amdgcn_exp2f(ml.x - nm);
-        mx = nm;
-      }
-    }
-  }
-  // combine across lanes: within 16-lane rows by DPP exchanges (the
-  // combination is symmetric, so both lanes of a pair hold the same bits),
-  // then the four rows' results, read as uniform values, in row order
-  auto combine = [&](float om, float os) __attribute__((always_inline)) {
-    const float nm = fmaxf(mx, om);
-    sm = nm == -INFINITY ? 0.0f
-                         : sm * __builtin_amdgcn_exp2f(mx - nm) + os * __builtin_amdgcn_exp2f(om - nm);
-    mx = nm;
-  };
-  combine(row_xchg<0xB1>(mx), row_xchg<0xB1>(sm));
-  combine(row_xchg<0x4E>(mx), row_xchg<0x4E>(sm));
-  combine(row_xchg<0x141>(mx), row_xchg<0x141>(sm));
-  combine(row_xchg<0x140>(mx), row_xchg<0x140>(sm));
-  {
-    float rm[4], rs[4];
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      rm[r] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(mx), 16 * r));
-      rs[r] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(sm), 16 * r));
-    }
-    mx = rm[0];
-    sm = rs[0];
-#pragma unroll
-    for (int r = 1; r < 4; ++r) combine(rm[r], rs[r]);
-  }
-  const float inv = 1.0f / fmaxf(sm, 1e-20f);
-  // lane l: weight 2^(m - M) / S of piece l
-  const float w_first = mine.y > 0.0f ? __builtin_amdgcn_exp2f(mine.x - mx) * inv : 0.0f;
-  float acc[PER];
-#pragma unroll
-  for (int i = 0; i < PER; ++i) acc[i] = 0.0f;
-  for (int k0 = 0; k0 < pc.n; k0 += NW * KW) {
-    if (k0 > 0) request(k0);
-    // lane l: weight of piece k0 + l (pieces below 64 from the pass above)
-    const bool held = k0 + NW * KW <= 64;
-    float wl = w_first;
-    if (!held) {
-      wl = 0.0f;
-      const int k = k0 + lane;
-      if (k < pc.n) {
-        const float2 ml = *(const float2 *)(a.part_ml + ((int64_t)pc.slot(k) * a.rows + row) * 2);
-        wl = ml.y > 0.0f ? __builtin_amdgcn_exp2f(ml.x - mx) * inv : 0.0f;
-      }
-    }
-#pragma unroll
-    for (int i = 0; i < KW; ++i) {
-      const int src_lane = held ? k0 + wv + NW * i : wv + NW * i;
-      const float wk = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(wl), src_lane));
-#pragma unroll
-      for (int e = 0; e < PER; ++e) acc[e] += wk * x[i][e];
-    }
-  }
-  if (wv > 0) {
-#pragma unroll
-    for (int e = 0; e < PER; ++e) s_acc[wv - 1][lane * PER + e] = acc[e];
-  }
-  __syncthreads();
-  if (wv != 0) return;
-  const int qi = row / a.gqa, h = kh * a.gqa + row % a.gqa;
-  uint16_t *o = a.out + (((int64_t)b * a.heads + h) * a.nq_stride + qi) * a.dim;
-#pragma unroll
-  for (int e = 0; e < PER; ++e) {
-    const int d = lane * PER + e;
-    float v = acc[e];
-#pragma unroll
-    for (int k = 0; k < NW - 1; ++k) v += s_acc[k][d];
-    if (d < a.dim) o[d] = float_to_bits(v, a.float_kind);
-  }
+  merge_unit<DP, NW>(a, (int)blockIdx.x);
 }
 
 template <int BITS, int DP, int G, int RB, int FK, int SLOTS, bool APPEND>
@@ -1954,6 +1731,16 @@ int attention_group(const Geo &g, int rows, bool append) { return group_of(g, ro
 
 bool append_fusable(const Geo &g, int rows) { return select_kernel(g, rows, true) != nullptr; }
 
+int device_cus() {
+  static std::atomic<int> known[64];
+  int dev = 0, cus = 0;
+  if (hipGetDevice(&dev) != hipSuccess) return -1;
+  if (dev < 64 && known[dev].load() > 0) return known[dev].load();
+  if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) return -1;
+  if (dev < 64) known[dev].store(cus);
+  return cus;
+}
+
 int attention_waves(const Geo &g, int rows) {
   const AttnKernel k = select_kernel(g, rows);
   if (!k) return -1;
@@ -1990,18 +1777,23 @@ hipError_t launch_attention(hipStream_t stream, const AttnArgs &a) {
 
 constexpr int64_t kMergeResidentWaves = 8192;
 
+// Waves per workgroup: enough for a segment's pieces, about waves / segments + 1,
+// to fit one round of 16 partial rows per wave (a single wave needs no LDS
+// reduction); two instead of four when four-wave workgroups would not all be
+// resident at once (about 8,192 waves on the device).
+int merge_waves(const MergeArgs &a) {
+  const int64_t units = (int64_t)a.batch * a.hk * a.rows;
+  const int64_t segments = (int64_t)a.batch * a.hk;
+  const int64_t pieces = (a.waves + segments - 1) / segments + 1;
+  const int nw = pieces <= 16 ? 1 : pieces <= 32 ? 2 : 4;
+  return nw == 4 && units * 4 > kMergeResidentWaves ? 2 : nw;
+}
+
 hipError_t launch_merge(hipStream_t stream, const MergeArgs &a) {
   const int64_t units = (int64_t)a.batch * a.hk * a.rows;  // one workgroup per (segment, row)
   if (units == 0 || a.waves <= 1) return hipSuccess;  // one run covers every segment whole
   if (units > 0x7FFFFFFF) return hipErrorInvalidValue;
-  // Waves per workgroup: enough for a segment's pieces, about waves /
-  // segments + 1, to fit one round of 16 partial rows per wave (a single wave
-  // needs no LDS reduction); two instead of four when four-wave workgroups
-  // would not all be resident at once (about 8,192 waves on the device).
-  const int64_t segments = (int64_t)a.batch * a.hk;
-  const int64_t pieces = (a.waves + segments - 1) / segments + 1;
-  int nw = pieces <= 16 ? 1 : pieces <= 32 ? 2 : 4;
-  if (nw == 4 && units * 4 > kMergeResidentWaves) nw = 2;
+  const int nw = merge_waves(a);
   const dim3 grid((unsigned)units), block(64 * nw);
 #define PKV_M(DP_)                                                                         \
   if (a.dp == DP_) {                                                                       \

@@ -59,6 +59,12 @@ struct AttnArgs {
   // the pool, writable) by the wave that attends the sequence's last tile.
   uint8_t *wpool = nullptr;
   const uint16_t *new_k = nullptr, *new_v = nullptr;
+  // Prefill kernel: the CUs to fill (0: no split) and the partials of spans cut
+  // into pieces (prefill_split): pieces per row block, then per piece the rows'
+  // (m, l) [block*S + piece][rows per block][2] and O^T as its lanes hold it.
+  int pre_cus = 0;
+  int32_t *pre_cnt = nullptr;
+  float *pre_ml = nullptr, *pre_acc = nullptr;
 };
 
 struct MergeArgs {
@@ -69,6 +75,19 @@ struct MergeArgs {
   const float *part_acc, *part_ml;
   uint16_t *out;
 };
+
+// Pieces the span of each row block is cut into when `blocks` prefill workgroups
+// (one per CU: LDS) would leave CUs idle: as many as fill the CUs once, or
+// twice where that is over 10% shorter (three pieces in two rounds of a grid
+// between half and two thirds of the CUs).  At most two pieces per CU (the
+// partials' space) and kMaxPrefillSplit per span.
+constexpr int kMaxPrefillSplit = 32;
+__host__ __device__ inline int prefill_split(int64_t blocks, int cus) {
+  if (blocks < 1 || blocks > cus) return 1;
+  const uint32_t once = (uint32_t)cus / (uint32_t)blocks, twice = 2 * (uint32_t)cus / (uint32_t)blocks;
+  const uint32_t s = 9 * twice > 20 * once ? twice : once;
+  return s < kMaxPrefillSplit ? (int)s : kMaxPrefillSplit;
+}
 
 struct QuantRowsArgs {
   const uint16_t *values;  // [rows][dim], float_kind
@@ -136,8 +155,17 @@ hipError_t launch_copy(hipStream_t stream, uint8_t *pool, int64_t num_pages, int
                        const int32_t *src, const int32_t *dst, int count);
 hipError_t launch_attention(hipStream_t stream, const AttnArgs &a);
 hipError_t launch_merge(hipStream_t stream, const MergeArgs &a);
+// Waves per merge workgroup.
+int merge_waves(const MergeArgs &a);
 // Query blocks wider than the decode kernel serves (chunked prefill).
 hipError_t launch_prefill(hipStream_t stream, const AttnArgs &a);
+// Row blocks per (sequence, KV head) and rows per block of the prefill kernel.
+int prefill_blocks(const Geo &g, int rows);
+int prefill_block_rows(const Geo &g);
+// The merges of a wide call in one launch: the decode parts' (`tiers` of
+// `tier`) and, with `prefill` (a.pre_cus > 0), the split prefill spans'.
+hipError_t launch_tail_merge(hipStream_t stream, const MergeArgs *tier, int tiers, const AttnArgs &a, bool prefill);
+int device_cus();
 // Resident waves of the attention kernel for this layout and row count on the
 // current device (CUs x workgroups per CU); <0 on error.
 int attention_waves(const Geo &g, int rows);

@@ -42,6 +42,7 @@
 // and masked.
 #include <type_traits>
 
+#include "pkv_merge.h"
 #include "pkv_mfma.h"
 
 namespace pkv {
@@ -103,13 +104,15 @@ __device__ __forceinline__ uint16_t bf16_bits_cvt(float x) {
   return __builtin_bit_cast(uint16_t, (__bf16)x);
 }
 
-__device__ __forceinline__ int prefill_width(const AttnArgs &a, int b) {
+template <typename Args>
+__device__ __forceinline__ int prefill_width(const Args &a, int b) {
   return a.widths ? (a.narrow_q > 0 && a.widths[b] <= a.narrow_q ? 0 : a.widths[b]) : a.nq;
 }
 
 // The k-th (from 0) sequence, in batch order, whose rows are live here
 // (live) or not (!live); -1 past the last.  Uniform; the whole wave calls.
-__device__ int nth_sequence(const AttnArgs &a, bool live, int k, int lane) {
+template <typename Args>
+__device__ int nth_sequence(const Args &a, bool live, int k, int lane) {
   int carry = 0;
   for (int c0 = 0; c0 < a.batch; c0 += 64) {
     const int idx = c0 + lane;
@@ -143,7 +146,8 @@ __device__ __forceinline__ void zero_row(uint16_t *o, int dim, int lane) {
 // while this MFMA-bound kernel leaves it idle instead of lingering in the
 // memory-side cache to be written back under the decode kernel that follows
 // (its launch: 88 -> 69 us in a mixed C2 + C5 batch).
-__device__ __forceinline__ void zero_share(const AttnArgs &a, int64_t z, int64_t zend, int tid,
+template <typename Args>
+__device__ __forceinline__ void zero_share(const Args &a, int64_t z, int64_t zend, int tid,
                                            int nthreads) {
   const int lane = tid & 63, wv = tid >> 6, nwaves = nthreads >> 6;
   const int64_t per_seq = (int64_t)a.g.hk * a.rows;
@@ -179,6 +183,70 @@ __device__ __forceinline__ void zero_share(const AttnArgs &a, int64_t z, int64_t
   }
 }
 
+// The grid's work: live (sequence, KV head) segments, row blocks per segment and
+// pieces per span; `share`: a mixed batch, whose dead rows are shared out too.
+struct PrefillGrid {
+  int nseg, nblk, split;
+  bool share;
+};
+
+template <int ROWS, bool SHARE>
+__device__ __forceinline__ PrefillGrid prefill_grid(const AttnArgs &a, int lane) {
+  PrefillGrid p;
+  p.nblk = (a.rows + ROWS - 1) / ROWS;
+  p.share = false;
+  int nseq = a.batch;
+  if constexpr (SHARE) {
+    int nlive = 0;
+    for (int c0 = 0; c0 < a.batch; c0 += 64) {
+      const int idx = c0 + lane;
+      nlive += wave_sum(idx < a.batch && prefill_width(a, idx) > 0 ? 1 : 0);
+    }
+    p.share = nlive > 0 && nlive < a.batch;
+    if (p.share) nseq = nlive;
+  }
+  p.nseg = nseq * a.g.hk;
+  p.split = a.pre_cus > 0 ? prefill_split((int64_t)p.nseg * p.nblk, a.pre_cus) : 1;
+  return p;
+}
+
+// Workgroup -> (segment, row block, piece).  Blocks of one segment read the same
+// pages: they go to one XCD (workgroups are dealt to the 8 XCDs round-robin),
+// so its span is fetched into one L2.  With a multiple of 8 segments XCD x
+// runs segments x, x + 8, ... (heavy segments that sit together in the batch
+// still spread over every XCD), the longest spans of all of them (a causal
+// chunk's last row blocks) first, so that the grid does not end on them: three
+// f16 prompts of 1,000 tokens (384 blocks of 1 to 8 stages on 256 CUs)
+// 78 -> 62 us.  Otherwise each XCD takes an eighth of the blocks, in segment order.
+__device__ __forceinline__ void prefill_item(const PrefillGrid &p, int bid, int &seg, int &rblk, int &piece) {
+  const int x = bid & 7;
+  int k = bid >> 3;
+  if ((p.nseg & 7) == 0) {
+    const int spx = p.nseg >> 3;
+    seg = x + 8 * (k % spx);
+    k /= spx;
+  } else {
+    const int total = p.nseg * p.nblk * p.split;
+    k += x * (total >> 3) + min(x, total & 7);
+    const int per = p.nblk * p.split;
+    seg = k / per;
+    k -= seg * per;
+  }
+  piece = k % p.split;
+  rblk = p.nblk - 1 - k / p.split;
+}
+
+// Pieces a span of `stages` stages is cut into where the row blocks of the grid
+// are too few for the CUs (prefill_split): at least kSplitStages stages each (a
+// piece costs its start-up and 130 KB of partials, written and read).  One
+// sequence's chunk of 500 tokens behind 8,000 (64 row blocks, 4 pieces each)
+// 295 -> 98 us of kernel plus 14 us of merge; batches with a row block per CU
+// keep whole spans and no merge.
+constexpr int kSplitStages = 2;
+__device__ __forceinline__ int prefill_pieces(int stages, int split) {
+  return max(1, min(split, stages / kSplitStages));
+}
+
 template <int BITS, int DP, int G, int FK, bool SHARE>
 __global__ __launch_bounds__(64 * kMaxPrefillWaves) void prefill_kernel(const AttnArgs a) {
   constexpr int kPrefillWaves = prefill_waves(DP);
@@ -207,6 +275,7 @@ __global__ __launch_bounds__(64 * kMaxPrefillWaves) void prefill_kernel(const At
   __shared__ __attribute__((aligned(16))) uint8_t s_valid[2][kStageTiles];
   __shared__ int s_lim[2][kPrefillWaves];
   __shared__ int64_t s_zero[SHARE ? 2 : 1];  // zero share: first row, end
+  __shared__ int s_item[3];  // pieces of the span, the block's piece, its partial
   __shared__ __attribute__((aligned(16))) uint16_t stage[2][I::ELEMS];
   // score metadata of the stage's K tiles (quantized pages)
   constexpr int SPG = BF16_BIAS ? 6 : bias_parts(NG);
@@ -218,11 +287,7 @@ __global__ __launch_bounds__(64 * kMaxPrefillWaves) void prefill_kernel(const At
   const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int col = lane & 15, jj = lane >> 4;
   const Geo &g = a.g;
-  // Work items.  Blocks of one (sequence, KV head) read the same pages: give
-  // them consecutive slots of one XCD (workgroups are dealt to the 8 XCDs
-  // round-robin) so the span is fetched into one L2.  XCD x runs segments
-  // x, x + 8, x + 16, ...: heavy segments that sit together in the batch still
-  // spread over every XCD.
+  // Work items (prefill_item).
   //
   // A mixed batch's sequences that the decode kernel serves (width 0 here)
   // only need zeros in their rows (the decode kernel, launched next, writes
@@ -234,38 +299,30 @@ __global__ __launch_bounds__(64 * kMaxPrefillWaves) void prefill_kernel(const At
   // times), and the rest of the grid exits at once.
   // (SHARE: the instantiation for mixed batches, launched when the decode
   // kernel serves some of the call's sequences; others carry none of it.)
-  const int nblk = (a.rows + ROWS - 1) / ROWS;
-  int bid = blockIdx.x;
+  const PrefillGrid pg = prefill_grid<ROWS, SHARE>(a, lane);
+  const int nblk = pg.nblk;
+  const int bid = blockIdx.x;
+  const int R = pg.nseg * nblk * pg.split;
+  if (bid >= R) return;
   int64_t zlo = 0, zhi = 0;  // zero rows (of the flattened dead-row space) this block writes
-  bool share = false;
-  int R = (int)gridDim.x;
+  const bool share = SHARE && pg.share;
   if constexpr (SHARE) {
-    int nlive = 0;
-    for (int c0 = 0; c0 < a.batch; c0 += 64) {
-      const int idx = c0 + lane;
-      nlive += wave_sum(idx < a.batch && prefill_width(a, idx) > 0 ? 1 : 0);
-    }
-    share = nlive > 0 && nlive < a.batch;
     if (share) {
-      R = nlive * g.hk * nblk;
-      if (bid >= R) return;
-      const int64_t Z = (int64_t)(a.batch - nlive) * g.hk * a.rows;
+      const int64_t Z = (int64_t)(a.batch - pg.nseg / g.hk) * g.hk * a.rows;
       zlo = (int64_t)bid * Z / R;
       zhi = (int64_t)(bid + 1) * Z / R;
     }
   }
-  const int span = R;
-  if (((span / nblk) & 7) == 0) {
-    const int x = bid & 7, k = bid >> 3;
-    bid = (x + 8 * (k / nblk)) * nblk + k % nblk;
-  }
-  const int seg = bid / nblk, rblk = bid % nblk;
+  int seg, rblk, piece;
+  prefill_item(pg, bid, seg, rblk, piece);
   const int b = share ? nth_sequence(a, true, seg / g.hk, lane) : seg / g.hk;
   const int kh = seg % g.hk;
   if (b < 0 || b >= a.batch) return;
   const int L = a.seq_lens[b];
   const int width = prefill_width(a, b);
   if (SHARE && width <= 0) {
+    if (piece == 0 && tid == 0 && pg.split > 1) a.pre_cnt[seg * nblk + rblk] = 1;  // nothing to merge
+    if (piece > 0) return;
     // no row of this sequence is live here (every sequence of the call is
     // left to the decode kernel): the block's rows are zeros, written
     // without the query loads and the span walk (elsewhere such rows take
@@ -425,9 +482,41 @@ __global__ __launch_bounds__(64 * kMaxPrefillWaves) void prefill_kernel(const At
   }
   tmax = __builtin_amdgcn_readfirstlane(tmax);
   tmin = __builtin_amdgcn_readfirstlane(tmin);
-  const int ntiles = tmax >= 0 ? tmax / PKV_TILE + 1 : 0;
-  const int clear_tiles = tmin == 0x7FFFFFFF ? 0 : (tmin + 1) / PKV_TILE;
-  const int nstages = (ntiles + kStageTiles - 1) / kStageTiles;
+  int ntiles = tmax >= 0 ? tmax / PKV_TILE + 1 : 0;
+  int clear_tiles = tmin == 0x7FFFFFFF ? 0 : (tmin + 1) / PKV_TILE;
+  int nstages = (ntiles + kStageTiles - 1) / kStageTiles;
+  int Lrel = L;  // tokens of the sequence, from the block's first stage on
+  int page0 = 0; // and its first page
+  // A piece of the span: everything below counts from its first tile (pieces
+  // start on page boundaries), so the stage loop holds no more than it does
+  // for a whole span; what the epilogue needs of the item waits in LDS.
+  if (pg.split > 1) {
+    constexpr int kAlign = kStageTiles < 8 ? 2 : 1;  // stages per 128 tokens (the largest page)
+    const int n = (nstages + kAlign - 1) / kAlign;
+    const int pieces = prefill_pieces(n, pg.split);
+    int s0 = 0, s1 = 0;
+    if (piece < pieces) {
+      s0 = n * piece / pieces * kAlign;
+      s1 = min(nstages, n * (piece + 1) / pieces * kAlign);
+    }
+    const int t0 = s0 * kStageTiles;
+    ntiles = max(0, min(ntiles, s1 * kStageTiles) - t0);
+    clear_tiles -= t0;
+    nstages = s1 - s0;
+    Lrel -= t0 * PKV_TILE;
+    page0 = t0 * PKV_TILE / g.page;
+#pragma unroll
+    for (int rb = 0; rb < RB; ++rb) lim[rb] -= lim[rb] < 0 ? 0 : t0 * PKV_TILE;  // < 0: nothing visible here
+    if (tid == 0) {
+      if (piece == 0) a.pre_cnt[seg * nblk + rblk] = pieces;
+      s_item[0] = pieces;
+      s_item[1] = piece;
+      s_item[2] = (seg * nblk + rblk) * pg.split + piece;
+    }
+  } else if (tid == 0) {
+    s_item[0] = 1;
+    s_item[1] = 0;
+  }
   const int tpp_shift = __builtin_ctz(g.page / PKV_TILE);
   const int tpp_mask = (1 << tpp_shift) - 1;
 
@@ -440,7 +529,8 @@ __global__ __launch_bounds__(64 * kMaxPrefillWaves) void prefill_kernel(const At
   // a VGPR and read with v_readlane made every lookup wait for all vector
   // loads in flight, the tile loads just issued included.)
   typedef __attribute__((address_space(4))) const int32_t cint32;  // read-only: scalar loads
-  cint32 *trow = (cint32 *)(a.table + (int64_t)b * a.max_pages);
+  cint32 *trow = (cint32 *)(a.table + (int64_t)b * a.max_pages + page0);
+  const int row_pages = a.max_pages - page0;
   int n_ok = 0, n_t = 0, n_tip = 0;  // the located tile
   const uint8_t *n_head = a.pool;
   // tile kStageTiles*s + wv of stage s -> (present, tile, head block, tile offset)
@@ -450,7 +540,7 @@ __global__ __launch_bounds__(64 * kMaxPrefillWaves) void prefill_kernel(const At
     n_tip = 0;
     if (n_t < ntiles) {
       const int p = n_t >> tpp_shift;
-      const int pid = p < a.max_pages ? trow[p] : -1;
+      const int pid = p < row_pages ? trow[p] : -1;
       if (pid >= 0 && pid < a.num_pages) {
         id = pid;
         n_tip = n_t & tpp_mask;
@@ -497,11 +587,11 @@ __global__ __launch_bounds__(64 * kMaxPrefillWaves) void prefill_kernel(const At
     uint16_t *img = stage[dst];
     const int r_ok = k_half ? k_ok : v_ok;
     const int tok0 = (k_half ? k_t : v_t) * PKV_TILE;
-    const bool whole = r_ok && tok0 + PKV_TILE <= L;  // uniform
-    const bool kvalid = r_ok && tok0 + col < L;
+    const bool whole = r_ok && tok0 + PKV_TILE <= Lrel;  // uniform
+    const bool kvalid = r_ok && tok0 + col < Lrel;
     bool vvalid[4];
 #pragma unroll
-    for (int e = 0; e < 4; ++e) vvalid[e] = r_ok && tok0 + 4 * jj + e < L;
+    for (int e = 0; e < 4; ++e) vvalid[e] = r_ok && tok0 + 4 * jj + e < Lrel;
     uint16_t *kdst = img + wv * I::KTILE + col * I::KROW + 8 * jj;
     uint16_t *vdst = img + I::K_ELEMS + col * I::VROW + 32 * (wv >> 1) + 8 * jj + 4 * (wv & 1);
     if constexpr (QUANT) {
@@ -865,6 +955,14 @@ __global__ __launch_bounds__(64 * kMaxPrefillWaves) void prefill_kernel(const At
   }
 
   // ---- epilogue: fold the 4 jj lanes of a column, normalise, write
+  // (the arguments it needs are read again here, through a pointer the compiler
+  // cannot trace to the kernel's own, instead of being held in scalar registers
+  // across the stage loop)
+  typedef __attribute__((address_space(4))) const AttnArgs LateArgs;
+  LateArgs *late = (LateArgs *)__builtin_amdgcn_kernarg_segment_ptr();
+  asm volatile("" : "+s"(late));
+  const int pieces = __builtin_amdgcn_readfirstlane(s_item[0]);
+  const int piece_of = __builtin_amdgcn_readfirstlane(s_item[1]);
 #pragma unroll
   for (int rb = 0; rb < RB; ++rb) {
     if constexpr (MSUM) {
@@ -873,28 +971,42 @@ __global__ __launch_bounds__(64 * kMaxPrefillWaves) void prefill_kernel(const At
       lsum[rb] += __shfl_xor(lsum[rb], 16, 64);
       lsum[rb] += __shfl_xor(lsum[rb], 32, 64);
     }
+    if (pieces > 1) {
+      // the piece's partial: (m, l) per row, O^T as the lanes hold it; rows
+      // that are not live leave zeros
+      if (piece_of >= pieces) continue;
+      const int64_t blk = s_item[2];
+      const int rb16 = wv * RB + rb;
+      const bool live = lim[rb] >= 0;
+      if (jj == 0)
+        *(float2 *)(late->pre_ml + (blk * ROWS + rb16 * 16 + col) * 2) = make_float2(m[rb], live ? lsum[rb] : 0.0f);
+      float *dst = late->pre_acc + (blk * (ROWS / 16) + rb16) * (16 * DP) + lane * 4;
+#pragma unroll
+      for (int n = 0; n < NB; ++n) *(f4 *)(dst + n * 256) = live ? O[rb][n] : f4{0.0f, 0.0f, 0.0f, 0.0f};
+      continue;
+    }
     const int row = rblk * ROWS + wv * 16 * RB + rb * 16 + col;
-    if (row >= a.rows) continue;
-    const int qi = row / a.gqa, h = kh * a.gqa + row % a.gqa;
+    if (row >= late->rows || piece_of > 0) continue;
+    const int qi = row / late->gqa, h = kh * late->gqa + row % late->gqa;
     // dead rows (past the chunk's width) ran the unmasked steps: write 0
     const float inv = lim[rb] < 0 ? 0.0f : 1.0f / fmaxf(lsum[rb], 1e-20f);
-    uint16_t *o = a.out + (((int64_t)b * a.heads + h) * a.nq + qi) * g.dim;
+    uint16_t *o = late->out + (((int64_t)b * late->heads + h) * late->nq + qi) * late->g.dim;
 #pragma unroll
     for (int n = 0; n < NB; ++n) {
       float v4[4];
 #pragma unroll
       for (int r = 0; r < 4; ++r) v4[r] = lim[rb] < 0 ? 0.0f : O[rb][n][r] * inv;
       const int d = 16 * n + 4 * jj;
-      if ((g.dim & 3) == 0 && d + 4 <= g.dim) {
-        u2 packed = {(uint32_t)float_to_bits(v4[0], g.float_kind) |
-                         ((uint32_t)float_to_bits(v4[1], g.float_kind) << 16),
-                     (uint32_t)float_to_bits(v4[2], g.float_kind) |
-                         ((uint32_t)float_to_bits(v4[3], g.float_kind) << 16)};
+      if ((late->g.dim & 3) == 0 && d + 4 <= late->g.dim) {
+        u2 packed = {(uint32_t)float_to_bits(v4[0], late->g.float_kind) |
+                         ((uint32_t)float_to_bits(v4[1], late->g.float_kind) << 16),
+                     (uint32_t)float_to_bits(v4[2], late->g.float_kind) |
+                         ((uint32_t)float_to_bits(v4[3], late->g.float_kind) << 16)};
         *(u2 *)(o + d) = packed;
       } else {
 #pragma unroll
         for (int r = 0; r < 4; ++r)
-          if (d + r < g.dim) o[d + r] = float_to_bits(v4[r], g.float_kind);
+          if (d + r < late->g.dim) o[d + r] = float_to_bits(v4[r], late->g.float_kind);
       }
     }
   }
@@ -902,7 +1014,90 @@ __global__ __launch_bounds__(64 * kMaxPrefillWaves) void prefill_kernel(const At
   // rows (stores issued before the stages would hold up the first tile
   // loads: vmcnt counts both, in order)
   if constexpr (SHARE) {
-    if (share) zero_share(a, s_zero[0], s_zero[1], tid, 64 * kPrefillWaves);
+    if (s_zero[1] > s_zero[0]) zero_share(*late, s_zero[0], s_zero[1], tid, 64 * kPrefillWaves);
+  }
+}
+
+// ---- merge of split spans ----------------------------------------------------------
+
+// One wave per 16 rows of a row block whose span was cut: every piece's (m, l),
+// then the pieces' O^T in the lanes' own layout (1 KiB loads, a piece's NB of
+// them in flight together), weighted by 2^(m - M) and normalised.
+template <int DP, bool SHARE>
+__device__ __forceinline__ void prefill_merge(const AttnArgs &a, int unit) {
+  constexpr int ROWS = prefill_rows(DP), RBLKS = ROWS / 16, NB = DP / 16;
+  const int lane = threadIdx.x & 63, col = lane & 15, jj = lane >> 4;
+  const int blk = unit / RBLKS, rb16 = unit % RBLKS;
+  const PrefillGrid pg = prefill_grid<ROWS, SHARE>(a, lane);
+  if (pg.split < 2 || blk >= pg.nseg * pg.nblk) return;
+  const int seg = blk / pg.nblk, rblk = blk % pg.nblk;
+  const int row = rblk * ROWS + rb16 * 16 + col;
+  const int pieces = min(a.pre_cnt[blk], pg.split);
+  if (pieces < 2 || rblk * ROWS + rb16 * 16 >= a.rows) return;
+  const int b = SHARE && pg.share ? nth_sequence(a, true, seg / a.g.hk, lane) : seg / a.g.hk;
+  const int kh = seg % a.g.hk;
+  if (b < 0 || b >= a.batch) return;
+  const float *ml = a.pre_ml + ((int64_t)blk * pg.split * ROWS + rb16 * 16 + col) * 2;
+  const float *src = a.pre_acc + ((int64_t)blk * pg.split * RBLKS + rb16) * (16 * DP) + lane * 4;
+  float M = -INFINITY;
+  for (int p = 0; p < pieces; ++p) {
+    const float2 x = *(const float2 *)(ml + (int64_t)p * ROWS * 2);
+    if (x.y != 0.0f) M = fmaxf(M, x.x);  // a piece without a visible token holds l = 0
+  }
+  float L = 0.0f;
+  f4 acc[NB];
+#pragma unroll
+  for (int n = 0; n < NB; ++n) acc[n] = f4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll 2
+  for (int p = 0; p < pieces; ++p) {
+    const float2 x = *(const float2 *)(ml + (int64_t)p * ROWS * 2);
+    f4 v[NB];
+#pragma unroll
+    for (int n = 0; n < NB; ++n) v[n] = *(const f4 *)(src + (int64_t)p * RBLKS * (16 * DP) + n * 256);
+    const float w = x.y != 0.0f ? __builtin_amdgcn_exp2f(x.x - M) : 0.0f;
+    L += w * x.y;
+#pragma unroll
+    for (int n = 0; n < NB; ++n) acc[n] += w * v[n];
+  }
+  if (row >= a.rows) return;
+  const int qi = row / a.gqa, h = kh * a.gqa + row % a.gqa;
+  const float inv = 1.0f / fmaxf(L, 1e-20f);
+  uint16_t *o = a.out + (((int64_t)b * a.heads + h) * a.nq + qi) * a.g.dim;
+#pragma unroll
+  for (int n = 0; n < NB; ++n) {
+    const int d = 16 * n + 4 * jj;
+    uint16_t e[4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) e[r] = float_to_bits(acc[n][r] * inv, a.g.float_kind);
+    if ((a.g.dim & 3) == 0 && d + 4 <= a.g.dim) {
+      *(u2 *)(o + d) = u2{(uint32_t)e[0] | ((uint32_t)e[1] << 16), (uint32_t)e[2] | ((uint32_t)e[3] << 16)};
+    } else {
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        if (d + r < a.g.dim) o[d + r] = e[r];
+    }
+  }
+}
+
+// Every merge of a wide call in one launch: workgroups [0, n0) the first decode
+// part's (segment, row) units, [n0, n0 + n1) the second's, the rest NW 16-row
+// units each of the split prefill spans.  (A launch with nothing to do still
+// costs 2 to 2.5 us on the stream, and the host cannot see which parts have
+// work: the widths live on the device.)
+struct TailArgs {
+  MergeArgs tier[2];
+  AttnArgs pre;
+  int n0, n1;
+};
+
+template <int DP, int NW, bool SHARE>
+__global__ __launch_bounds__(64 * NW) void tail_merge_kernel(const TailArgs a) {
+  const int u = (int)blockIdx.x;
+  if (u < a.n0 + a.n1) {
+    merge_unit<DP, NW>(a.tier[u < a.n0 ? 0 : 1], u < a.n0 ? u : u - a.n0);
+  } else {
+    const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    prefill_merge<DP, SHARE>(a.pre, (u - a.n0 - a.n1) * NW + wv);
   }
 }
 
@@ -929,16 +1124,69 @@ static PrefillKernel select_prefill(const Geo &g) {
   return nullptr;
 }
 
+int prefill_block_rows(const Geo &g) { return prefill_rows(g.dp); }
+int prefill_blocks(const Geo &g, int rows) { return (rows + prefill_rows(g.dp) - 1) / prefill_rows(g.dp); }
+
 hipError_t launch_prefill(hipStream_t stream, const AttnArgs &a) {
   // sequences left to the decode kernel: the instantiation that shares their zero rows out
-  const PrefillKernel k = a.widths && a.narrow_q > 0 ? select_prefill<true>(a.g) : select_prefill<false>(a.g);
+  const bool share = a.widths && a.narrow_q > 0;
+  const PrefillKernel k = share ? select_prefill<true>(a.g) : select_prefill<false>(a.g);
   if (!k) return hipErrorInvalidValue;
-  const int rows_per_block = prefill_rows(a.g.dp);
-  const int64_t blocks = (int64_t)a.batch * a.g.hk * ((a.rows + rows_per_block - 1) / rows_per_block);
+  int64_t blocks = (int64_t)a.batch * a.g.hk * prefill_blocks(a.g, a.rows);
   if (blocks == 0) return hipSuccess;
+  if (a.pre_cus > 0) {
+    // (the live sequences of a mixed batch, and so the split, are known on the
+    // device only: the grid covers any number of them; workgroups past the
+    // pieces exit at once, but each needs a CU's LDS to start, so there are no
+    // more than that)
+    const int64_t per_seq = blocks / a.batch;
+    int64_t most = share ? blocks : blocks * prefill_split(blocks, a.pre_cus);
+    for (int64_t n = per_seq; share && n <= blocks && n <= a.pre_cus; n += per_seq) {
+      const int64_t items = n * prefill_split(n, a.pre_cus);
+      most = items > most ? items : most;
+    }
+    blocks = most;
+  }
   if (blocks > 0x7FFFFFFF) return hipErrorInvalidValue;
   hipLaunchKernelGGL(k, dim3((unsigned)blocks), dim3(64 * prefill_waves(a.g.dp)), 0, stream, a);
   return hipGetLastError();
+}
+
+hipError_t launch_tail_merge(hipStream_t stream, const MergeArgs *tier, int tiers, const AttnArgs &a, bool prefill) {
+  TailArgs t;
+  int64_t n[2] = {0, 0};
+  int nw = 1;
+  for (int i = 0; i < tiers; ++i) {
+    t.tier[i] = tier[i];
+    n[i] = tier[i].waves > 1 ? (int64_t)tier[i].batch * tier[i].hk * tier[i].rows : 0;
+    const int w = merge_waves(tier[i]);
+    if (n[i] > 0 && w > nw) nw = w;
+  }
+  t.pre = a;
+  int64_t units = 0;
+  if (prefill) {
+    // row blocks that can be split: those of a grid of at most pre_cus blocks
+    int64_t blocks = (int64_t)a.batch * a.g.hk * prefill_blocks(a.g, a.rows);
+    if (blocks > a.pre_cus) blocks = a.widths && a.narrow_q > 0 ? a.pre_cus : 0;
+    units = (blocks * (prefill_rows(a.g.dp) / 16) + nw - 1) / nw;
+  }
+  const int64_t grid = n[0] + n[1] + units;
+  if (grid == 0) return hipSuccess;
+  if (grid > 0x7FFFFFFF) return hipErrorInvalidValue;
+  t.n0 = (int)n[0];
+  t.n1 = (int)n[1];
+  const bool share = a.widths && a.narrow_q > 0;
+  const dim3 g((unsigned)grid), block(64 * nw);
+#define PKV_T(DP_, NW_)                                                                                      \
+  if (a.g.dp == DP_ && nw == NW_) {                                                                          \
+    if (share) hipLaunchKernelGGL((tail_merge_kernel<DP_, NW_, true>), g, block, 0, stream, t);              \
+    else hipLaunchKernelGGL((tail_merge_kernel<DP_, NW_, false>), g, block, 0, stream, t);                   \
+    return hipGetLastError();                                                                                \
+  }
+  PKV_T(64, 1) PKV_T(64, 2) PKV_T(64, 4) PKV_T(128, 1) PKV_T(128, 2) PKV_T(128, 4)
+  PKV_T(256, 1) PKV_T(256, 2) PKV_T(256, 4)
+#undef PKV_T
+  return hipErrorInvalidValue;
 }
 
 }  // namespace pkv

@@ -200,11 +200,19 @@ def paged_attention(fmt: PageFormat, pool, queries, block_table, seq_lens, *, sc
     lens = _i32(seq_lens, device)
     if waves <= 0:
         waves = default_waves(fmt, heads, decode_queries(fmt, heads, nq) or nq, batch)
-    need = workspace_bytes(fmt, heads, nq, waves)
+    wide = decode_queries(fmt, heads, nq) != nq
+    if workspace is None and wide:
+        # room for split prefill spans too; the stream's own memory, since wide
+        # calls on other streams or threads may overlap this one
+        need = int(nat.load().pkv_attention_batch_workspace_bytes(fmt.c_layout, heads, nq, batch,
+                                                                  waves))
+    else:
+        need = workspace_bytes(fmt, heads, nq, waves)
     if need < 0:
         nat.check(nat.PKV_INVALID_ARGUMENT, "paged attention workspace")
     if workspace is None:
-        workspace = attention_workspace(device, need)
+        workspace = (torch.empty(max(need, 256), dtype=torch.uint8, device=device) if wide
+                     else attention_workspace(device, need))
     elif workspace.device != device or workspace.dtype != torch.uint8 or \
             not workspace.is_contiguous():
         raise ValueError("attention workspace must be a contiguous uint8 tensor on the "
