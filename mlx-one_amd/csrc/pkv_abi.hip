@@ -63,12 +63,13 @@ int64_t attention_runs(const pkv_geometry &g, int64_t rows, int64_t waves, bool 
   return std::max<int64_t>(1, waves / pkv::attention_group(pkv::to_geo(g), (int)rows, append));
 }
 
-// Partial space of a launch; `append` unknown (the public sizing query): the
-// larger of the forms the shape has.
+// Partial space of a launch; `append` unknown (the public sizing query): one run
+// per wave where the shape has a fused single-token form (more than either
+// form's runs need: the size callers have always been given).
 WorkspaceParts workspace_parts(const pkv_geometry &g, int64_t rows, int64_t waves, int append = -1) {
   int64_t runs = attention_runs(g, rows, waves, append > 0);
   if (append < 0 && pkv::append_fusable(pkv::to_geo(g), (int)rows))
-    runs = std::max(runs, attention_runs(g, rows, waves, true));
+    runs = std::max<int64_t>(runs, waves);
   const int64_t slots = (int64_t)pkv::kSlotsPerWave * runs;
   WorkspaceParts w;
   w.ml = 0;

@@ -87,9 +87,11 @@ constexpr bool kDequantRows = true;
 // Waves per run: the kernels for 5-8 rows (two column slots) and 17-32 rows
 // (two row blocks) per KV head give each run of the split to a workgroup of
 // this many waves, which share its iterations round robin and combine their
-// states in LDS at each piece's end; the others (and the fused single-token
-// append) run one wave per run.
-constexpr int run_waves(int rb, int slots, bool append) { return !append && (rb == 2 || slots == 2) ? 4 : 1; }
+// states in LDS at each piece's end; the others run one wave per run.  The fused
+// single-token append runs as its shape does without it: the wave that takes a
+// piece's last iteration appends (8 sequences of 32K 4-bit tokens, 8 rows per KV
+// head: 50.5 us at one wave per run, 38.4 grouped).
+constexpr int run_waves(int rb, int slots) { return rb == 2 || slots == 2 ? 4 : 1; }
 
 template <int DP, int NW>
 __global__ __launch_bounds__(64 * NW) void merge_kernel(const MergeArgs a) {
@@ -97,7 +99,7 @@ __global__ __launch_bounds__(64 * NW) void merge_kernel(const MergeArgs a) {
 }
 
 template <int BITS, int DP, int G, int RB, int FK, int SLOTS, bool APPEND>
-__global__ __launch_bounds__(64 * run_waves(RB, SLOTS, APPEND))
+__global__ __launch_bounds__(64 * run_waves(RB, SLOTS))
 __attribute__((amdgpu_waves_per_eu(min_waves_per_simd(BITS, DP, G, RB, SLOTS)))) void attn_kernel(
     const AttnArgs a) {
   using C = Cfg<BITS, DP, G, RB, FK, SLOTS>;
@@ -133,7 +135,7 @@ __attribute__((amdgpu_waves_per_eu(min_waves_per_simd(BITS, DP, G, RB, SLOTS))))
   // piece loop instead of hoisting them all and pinning them in registers.
   // Runs of GW waves (GW > 1): wave wk of the workgroup takes iterations wk,
   // wk + GW, ... of each piece of the run.
-  constexpr int GW = run_waves(RB, SLOTS, APPEND);
+  constexpr int GW = run_waves(RB, SLOTS);
   const int wk = GW > 1 ? __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6) : 0;
   int lane = threadIdx.x & 63;
   int col, jj, slot_l, rowc;  // slot_l: this lane's column slot; rowc: its row within the slot
@@ -664,7 +666,8 @@ __attribute__((amdgpu_waves_per_eu(min_waves_per_simd(BITS, DP, G, RB, SLOTS))))
     const int niters = max(1, (ntl + SLOTS - 1) / SLOTS);
     int cwin = cta >> tpp_shift;
     int cmask;
-    const bool appends = APPEND && ctb == cnt && cL > 0;  // the piece holds the segment's last tile
+    // the piece holds the segment's last tile, this wave its last iteration
+    const bool appends = APPEND && ctb == cnt && cL > 0 && (GW == 1 || (niters - 1) % GW == wk);
     {
       u4 raw[RB][KB];
       int qp[RB];
@@ -1721,10 +1724,9 @@ bool decode_serves(const Geo &g, int rows) { return select_kernel(g, rows) != nu
 // (two past 16 rows) and column slots (4, 2 or 1 up to 4, 8 and 16 rows, as
 // fit_slots leaves them); the VALU decode kernel runs one wave per run.
 static int group_of(const Geo &g, int rows, bool append = false) {
-  if (append) return 1;
-  if (rows <= 4 && g_decode_kernel.load() == kDecodeValu && select_valu(g)) return 1;
+  if (!append && rows <= 4 && g_decode_kernel.load() == kDecodeValu && select_valu(g)) return 1;
   const int req = rows <= 4 ? 4 : rows <= 8 ? 2 : 1;
-  return run_waves(rows > 16 ? 2 : 1, fit_slots(g.bits, g.dp, g.bits == 16 ? 32 : g.group, req), append);
+  return run_waves(rows > 16 ? 2 : 1, fit_slots(g.bits, g.dp, g.bits == 16 ? 32 : g.group, req));
 }
 
 int attention_group(const Geo &g, int rows, bool append) { return group_of(g, rows, append); }
@@ -1765,7 +1767,10 @@ int attention_waves(const Geo &g, int rows) {
 // the new token before its first tiles (C2: 67.8 us against 69.0 at 8).
 // A run of a grouped kernel (GW waves) moves GW tiles in a wave's tile time,
 // so its lead counts GW times as many tiles.
-int attention_lead(const Geo &g, int rows, bool append) { return append ? 16 : 8 * group_of(g, rows, append); }
+int attention_lead(const Geo &g, int rows, bool append) {
+  const int gw = group_of(g, rows, append);
+  return append && gw == 1 ? 16 : 8 * gw;
+}
 
 hipError_t launch_attention(hipStream_t stream, const AttnArgs &a) {
   const AttnKernel k = select_kernel(a.g, a.rows, a.new_k != nullptr);
