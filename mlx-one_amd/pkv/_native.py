@@ -85,6 +85,8 @@ _lib = None
 def load(path=None):
     """Load libpkv.so and bind every exported symbol (idempotent)."""
     global _lib
+    if path is None and _lib is not None:  # bound once, never replaced
+        return _lib
     with _lock:
         if _lib is not None and path is None:
             return _lib
@@ -126,10 +128,21 @@ def check(code, what):
 
 
 def ptr(tensor):
-    return None if tensor is None else ctypes.c_void_p(tensor.data_ptr())
+    """The tensor's device address, as the pointer arguments take it (None: NULL)."""
+    return None if tensor is None else tensor.data_ptr()
+
+
+_torch = None
 
 
 def stream_handle(device=None):
-    import torch
+    """The current stream of ``device`` (a torch device; default: the current one)."""
+    global _torch
+    if _torch is None:
+        import torch
 
-    return ctypes.c_void_p(torch.cuda.current_stream(device).cuda_stream)
+        _torch = torch
+    index = device.index if isinstance(device, _torch.device) else None
+    if index is None:
+        return _torch.cuda.current_stream(device).cuda_stream
+    return _torch._C._cuda_getCurrentRawStream(index)

@@ -10,6 +10,7 @@ from __future__ import annotations
 
 import math
 from dataclasses import dataclass
+from functools import cached_property
 
 import torch
 
@@ -42,16 +43,17 @@ class PageFormat:
         if self.page_bytes < 0:
             nat.check(nat.PKV_UNSUPPORTED, "page layout")
 
-    @property
+    # (computed once per format: every call passes them)
+    @cached_property
     def c_layout(self):
         return nat.Layout(self.num_kv_heads, self.head_dim, self.page_tokens, self.bits,
                           self.group_size if self.bits != 16 else 32, FLOAT_KINDS[self.dtype])
 
-    @property
+    @cached_property
     def page_bytes(self):
         return int(nat.load().pkv_page_bytes(self.c_layout))
 
-    @property
+    @cached_property
     def stored_dim(self):
         return int(nat.load().pkv_stored_dim(self.c_layout))
 
@@ -76,6 +78,8 @@ def _i32(x, device):
     if x is None:
         return None
     if isinstance(x, torch.Tensor):
+        if x.dtype is torch.int32 and x.device == device and x.is_contiguous():
+            return x
         t = x.to(device=device, dtype=torch.int32)
     else:
         t = torch.as_tensor(x, dtype=torch.int32).to(device)
@@ -132,6 +136,7 @@ def select_decode_kernel(kind):
     if kind not in DECODE_KERNELS:
         raise ValueError(f"decode kernel must be one of {sorted(DECODE_KERNELS)}")
     previous = int(nat.load().pkv_select_decode_kernel(DECODE_KERNELS[kind]))
+    _PLANS.clear()
     if previous < 0:
         nat.check(previous, "select decode kernel")
     return {v: k for k, v in DECODE_KERNELS.items()}[previous]
@@ -161,6 +166,37 @@ def workspace_bytes(fmt: PageFormat, num_heads, num_queries, waves):
                                                           waves))
 
 
+# (waves, workspace bytes) of a call shape with default waves: a few integers
+# per format, heads, queries, batch and device, as the library computed them
+# (cleared when the decode kernel changes, and when it holds many shapes).
+_PLANS = {}
+_MAX_PLANS = 4096
+
+
+def _plan(fmt, heads, nq, batch, device, wide=False):
+    """The default waves of a call and the workspace it runs best with."""
+    key = (fmt, heads, nq, batch, device)
+    plan = _PLANS.get(key)
+    if plan is None:
+        waves = default_waves(fmt, heads, decode_queries(fmt, heads, nq) or nq, batch)
+        plan = (waves, _workspace_need(fmt, heads, nq, batch, waves, wide))
+        if len(_PLANS) >= _MAX_PLANS:
+            _PLANS.clear()
+        _PLANS[key] = plan
+    return plan
+
+
+def _workspace_need(fmt, heads, nq, batch, waves, wide):
+    if wide:
+        need = int(nat.load().pkv_attention_batch_workspace_bytes(fmt.c_layout, heads, nq, batch,
+                                                                  waves))
+    else:
+        need = workspace_bytes(fmt, heads, nq, waves)
+    if need < 0:
+        nat.check(nat.PKV_INVALID_ARGUMENT, "paged attention workspace")
+    return need
+
+
 # One attention workspace per device, grown on demand; calls on one stream
 # share it (each call's partials are merged before the next call starts).
 _WORKSPACES = {}
@@ -168,7 +204,7 @@ _WORKSPACES = {}
 
 def attention_workspace(device, nbytes):
     """A workspace of at least ``nbytes`` on ``device`` (cached, grown on demand)."""
-    key = torch.device(device)
+    key = device if isinstance(device, torch.device) else torch.device(device)
     ws = _WORKSPACES.get(key)
     if ws is None or ws.numel() < nbytes:
         ws = torch.empty(max(int(nbytes), 256), dtype=torch.uint8, device=key)
@@ -198,18 +234,13 @@ def paged_attention(fmt: PageFormat, pool, queries, block_table, seq_lens, *, sc
     device = queries.device
     table = _i32(block_table, device)
     lens = _i32(seq_lens, device)
-    if waves <= 0:
-        waves = default_waves(fmt, heads, decode_queries(fmt, heads, nq) or nq, batch)
+    # a wide call has room for split prefill spans too, in the stream's own
+    # memory: wide calls on other streams or threads may overlap this one
     wide = decode_queries(fmt, heads, nq) != nq
-    if workspace is None and wide:
-        # room for split prefill spans too; the stream's own memory, since wide
-        # calls on other streams or threads may overlap this one
-        need = int(nat.load().pkv_attention_batch_workspace_bytes(fmt.c_layout, heads, nq, batch,
-                                                                  waves))
+    if waves <= 0:
+        waves, need = _plan(fmt, heads, nq, batch, device, wide)
     else:
-        need = workspace_bytes(fmt, heads, nq, waves)
-    if need < 0:
-        nat.check(nat.PKV_INVALID_ARGUMENT, "paged attention workspace")
+        need = _workspace_need(fmt, heads, nq, batch, waves, wide)
     if workspace is None:
         workspace = (torch.empty(max(need, 256), dtype=torch.uint8, device=device) if wide
                      else attention_workspace(device, need))
@@ -255,10 +286,9 @@ def append_paged_attention(fmt: PageFormat, pool, keys, values, queries, block_t
     table = _i32(block_table, device)
     lens = _i32(seq_lens, device)
     if waves <= 0:
-        waves = default_waves(fmt, heads, 1, batch)
-    need = workspace_bytes(fmt, heads, 1, waves)
-    if need < 0:
-        nat.check(nat.PKV_INVALID_ARGUMENT, "paged attention workspace")
+        waves, need = _plan(fmt, heads, 1, batch, device)
+    else:
+        need = _workspace_need(fmt, heads, 1, batch, waves, False)
     if workspace is None:
         workspace = attention_workspace(device, need)
     elif workspace.device != device or workspace.dtype != torch.uint8 or \
