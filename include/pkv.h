@@ -120,7 +120,11 @@ int pkv_append_quantize(void *stream, const pkv_layout *layout, void *pool, int6
  *                 when t <= q_pos (paged_attention.py:81)
  *  widths       : [batch] real query rows (rows q >= widths[b] output 0), or NULL
  *  scale        : softmax scale
- *  waves        : work waves; <= 0 picks pkv_attention_default_waves(...)
+ *  waves        : work waves; <= 0 leaves the choice to the library:
+ *                 pkv_attention_default_waves(...), or, where the block table
+ *                 holds a few hundred tokens per sequence, one run per (sequence,
+ *                 KV head) with no partials, or grouped runs for few segments
+ *                 (the workspace is checked against the default waves' all the same)
  *  workspace    : device scratch of pkv_attention_workspace_bytes(...) bytes
  *                 (calls sharing one workspace must not overlap)
  *  out          : [batch][num_heads][num_queries][head_dim], float_kind
@@ -137,8 +141,8 @@ int pkv_paged_attention(void *stream, const pkv_layout *layout, const void *pool
  * pkv_append_quantize with tokens = 1 at position seq_lens[b] - 1) and
  * attend its one query (as pkv_paged_attention with num_queries = 1, q_pos
  * NULL, widths NULL), in one launch where the decode kernel serves the shape
- * (quantized pages, at most 8 query rows per KV head): the wave that attends
- * a sequence's last tile quantizes the new token, stores it and uses it.
+ * (at most 8 query rows per KV head): the wave that attends a sequence's last
+ * tile quantizes the new token, stores it and uses it.
  * Other shapes run the append and the attention as two launches.  Replaces
  * the append-then-attend pair of PagedBatchCache.attend (engine/paged.py:
  * 260-263) for a decode step; pages and output equal the two separate calls'
@@ -213,7 +217,7 @@ int pkv_read_probe(void *stream, const pkv_layout *layout, const void *pool, int
  * prefill kernel).  <0 on error. */
 int32_t pkv_attention_waves(const pkv_layout *layout, int32_t num_heads, int32_t num_queries);
 
-/* The `waves` pkv_paged_attention uses when given waves <= 0: the resident
+/* The `waves` pkv_paged_attention sizes its work by when given waves <= 0: the resident
  * waves, or half of them (one per SIMD) for decode rows (<= 4 query rows per
  * KV head) on the MFMA decode kernel when the batch has at most a quarter as
  * many (sequence, KV head) segments as resident waves.  <0 on error. */

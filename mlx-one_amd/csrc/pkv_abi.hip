@@ -68,7 +68,7 @@ int64_t attention_runs(const pkv_geometry &g, int64_t rows, int64_t waves, bool 
 // form's runs need: the size callers have always been given).
 WorkspaceParts workspace_parts(const pkv_geometry &g, int64_t rows, int64_t waves, int append = -1) {
   int64_t runs = attention_runs(g, rows, waves, append > 0);
-  if (append < 0 && pkv::append_fusable(pkv::to_geo(g), (int)rows))
+  if (append < 0 && g.bits != 16 && pkv::append_fusable(pkv::to_geo(g), (int)rows))
     runs = std::max<int64_t>(runs, waves);
   const int64_t slots = (int64_t)pkv::kSlotsPerWave * runs;
   WorkspaceParts w;
@@ -118,6 +118,35 @@ int cached_waves(const pkv_geometry &geo, int rows) {
   const int w = pkv::attention_waves(pkv::to_geo(geo), rows);
   if (w > 0) cache[{dev, key}] = w;
   return w;
+}
+
+// How a decode call whose waves are left to the library runs.
+struct RunForm {
+  int group;  // waves per run of the grouped form where the shape's own is one wave (else 0)
+  int whole;  // one run per (sequence, KV head) segment: no partials, no merge launch
+};
+
+// Whole segments where the block table holds at most four iterations of a
+// four-wave run (4 x 4 waves x 16 tokens x column slots): the launch then takes
+// 7-12 us against 10-20 us for the split and its merge (300 tokens of 8-bit
+// pages, 4 rows per KV head: 10.6 us against 13.9 at 4 sequences, 14.1 against
+// 19.6 at 48; f16 pages, 500 tokens: 8.1 against 11.4), and past it longer (2,000
+// tokens: 21.5 against 14.9).  With four slots the fourth iteration (1,000
+// tokens) pays only when there are many segments (15.1 against 14.3 us at 4
+// sequences x 8 heads, 23.1 against 25.2 at 48).
+// Grouped runs where a segment would be cut into 128 pieces or more: a quarter as
+// many to merge (1 sequence x 8 heads of 16,000 tokens 19.5 -> 17.1 us, 2 heads
+// of 30,000 28.2 -> 16.5); at 64 pieces the longer lead of a group costs more
+// than the merge saves (2 sequences x 8 heads of 8,000: 17.4 against 19.5).
+RunForm run_form(const pkv_geometry &g, int rows, int64_t segments, int64_t table_tokens, int waves, bool append) {
+  const pkv::Geo geo = pkv::to_geo(g);
+  if (rows <= 4 && pkv::decode_kernel() == pkv::kDecodeValu) return {0, 0};
+  const int own = pkv::attention_group(geo, rows, append), four = pkv::attention_group_waves();
+  const int group = own > 1 ? 0 : four, slots = pkv::attention_slots(geo, rows);
+  const int iterations = slots == 4 && segments < 96 ? 3 : 4;
+  if (table_tokens <= (int64_t)iterations * 16 * slots * four) return {group, 1};
+  if (group && segments * 128 <= waves) return {group, 0};
+  return {0, 0};
 }
 
 // Most queries per sequence the split-K decode kernel serves at this GQA
@@ -439,6 +468,15 @@ int paged_attention_impl(void *stream, const pkv_layout *layout, const void *poo
     a.narrow_q = t.hi;
     a.waves = (int)attention_runs(geo, a.rows, t.waves, fused != nullptr);
     a.lead = pkv::attention_lead(a.g, a.rows, fused != nullptr);
+    if (!wide && waves <= 0) {
+      const RunForm f = run_form(geo, a.rows, (int64_t)batch * geo.hk, (int64_t)max_pages * geo.page, t.waves,
+                                 fused != nullptr);
+      a.group = f.group;
+      a.seg_runs = f.whole;
+      if (f.whole) a.waves = (int)((int64_t)batch * geo.hk);
+      else if (f.group) a.waves = std::max(1, t.waves / f.group);
+      if (f.group) a.lead = pkv::attention_group_lead();
+    }
     a.part_ml = (float *)((char *)workspace + part_base[i] + t.ws.ml);
     a.part_acc = (float *)((char *)workspace + part_base[i] + t.ws.acc);
     if (fused) {
@@ -468,7 +506,7 @@ int paged_attention_impl(void *stream, const pkv_layout *layout, const void *poo
     m.part_acc = a.part_acc;
     m.part_ml = a.part_ml;
     m.out = (uint16_t *)out;
-    if (together) continue;
+    if (together || a.seg_runs) continue;
     if (int rc = check_launch(pkv::launch_merge((hipStream_t)stream, m), "merge launch")) return rc;
   }
   if (together)

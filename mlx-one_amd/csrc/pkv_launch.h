@@ -49,7 +49,11 @@ struct AttnArgs {
   int max_pages;
   const int32_t *seq_lens, *q_pos, *widths;
   float scale_log2;  // softmax scale * log2(e)
-  int waves;         // work waves (grid size)
+  int waves;         // runs (grid size)
+  // Waves per run where the launch asks for the grouped form of a kernel that
+  // otherwise runs one wave per run (else 0), and whether run w is segment w,
+  // whole, instead of an equal share of the tiles (no partials, no merge).
+  int group = 0, seg_runs = 0;
   int lead;          // tiles of start-up cost charged ahead of each segment in the split
   float *part_acc;   // [2*waves][rows][DP]
   float *part_ml;    // [2*waves][rows][2]
@@ -176,11 +180,16 @@ int attention_group(const Geo &g, int rows, bool append);
 // Lead tiles the decode split charges per segment for `rows` query rows per KV
 // head (more for a launch that fuses the single-token append).
 int attention_lead(const Geo &g, int rows, bool append);
+// Waves per run and lead tiles of the grouped form every decode shape also has.
+int attention_group_waves();
+// Column slots (tiles per iteration of a wave) of the shape's kernel.
+int attention_slots(const Geo &g, int rows);
+int attention_group_lead();
 // Whether the split-K decode kernel serves this many rows per KV head (else
 // launch_prefill does, with no workspace and no merge).
 bool decode_serves(const Geo &g, int rows);
 // Whether the decode kernel fuses the single-token append for this layout and
-// row count (quantized pages, at most 8 rows per KV head).
+// row count (at most 8 rows per KV head).
 bool append_fusable(const Geo &g, int rows);
 // Decode kernel for <= 4 rows per KV head over quantized pages (head_dim <=
 // 128): process-wide; select returns the previous choice.

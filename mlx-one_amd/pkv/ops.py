@@ -186,6 +186,14 @@ def _plan(fmt, heads, nq, batch, device, wide=False):
     return plan
 
 
+def split_waves(fmt, heads, nq, batch, device):
+    """The default waves, to be passed explicitly: the call then always runs the
+    equal split over them, whatever its block table's width -- the arenas' calls
+    give the same bits from host tables (as wide as the batch) and from the
+    device's (as wide as ``max_tokens``)."""
+    return _plan(fmt, heads, nq, batch, device, decode_queries(fmt, heads, nq) != nq)[0]
+
+
 def _workspace_need(fmt, heads, nq, batch, waves, wide):
     if wide:
         need = int(nat.load().pkv_attention_batch_workspace_bytes(fmt.c_layout, heads, nq, batch,
@@ -218,7 +226,8 @@ def paged_attention(fmt: PageFormat, pool, queries, block_table, seq_lens, *, sc
 
     ``seq_lens`` counts the tokens in each sequence's cache (after the
     append) and stays on the device: the decode kernel shares the tiles of
-    all sequences out over ``waves`` waves (default: ``default_waves``);
+    all sequences out over ``waves`` waves (default 0: ``default_waves``, or
+    the library's form for short block tables and few segments);
     query blocks past 32 rows per KV head run on the prefill kernel -- and
     in a mixed batch (``widths`` given), the sequences narrow enough for the
     decode kernel still go to it, in the same call (``waves`` then sizes that
@@ -239,6 +248,8 @@ def paged_attention(fmt: PageFormat, pool, queries, block_table, seq_lens, *, sc
     wide = decode_queries(fmt, heads, nq) != nq
     if waves <= 0:
         waves, need = _plan(fmt, heads, nq, batch, device, wide)
+        if not wide:
+            waves = 0  # the library's choice, within the workspace of its default waves
     else:
         need = _workspace_need(fmt, heads, nq, batch, waves, wide)
     if workspace is None:
@@ -270,9 +281,10 @@ def append_paged_attention(fmt: PageFormat, pool, keys, values, queries, block_t
     """One single-token step: append ``keys``/``values [B, HK, 1, D]`` at
     position ``seq_lens - 1`` (``seq_lens`` counts the tokens after the
     append) and attend ``queries [B, H, 1, D]`` -- one launch where the decode
-    kernel serves the shape (quantized pages, at most 8 query rows per KV
-    head), else an append launch and the attention.  Pages and output equal
-    ``append_quantize`` followed by ``paged_attention`` bit for bit."""
+    kernel serves the shape (at most 8 query rows per KV head), else an
+    append launch and the attention.  Pages equal ``append_quantize``'s bit
+    for bit, outputs ``paged_attention``'s within its rounding (its split may
+    cut the tiles elsewhere)."""
     if queries.dim() != 4 or queries.shape[2] != 1:
         raise ValueError("queries must be [B, H, 1, D]")
     batch, heads, _, dim = queries.shape
@@ -286,7 +298,7 @@ def append_paged_attention(fmt: PageFormat, pool, keys, values, queries, block_t
     table = _i32(block_table, device)
     lens = _i32(seq_lens, device)
     if waves <= 0:
-        waves, need = _plan(fmt, heads, 1, batch, device)
+        waves, need = 0, _plan(fmt, heads, 1, batch, device)[1]
     else:
         need = _workspace_need(fmt, heads, 1, batch, waves, False)
     if workspace is None:

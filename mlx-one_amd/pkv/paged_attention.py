@@ -79,5 +79,6 @@ def paged_attention(queries, rows, positions, widths, *, scale, _device_meta=Non
         dtype = queries.dtype
         q = queries.to(device, pool.fmt.dtype)
         out = ops.paged_attention(pool.fmt, pool.buffer, q, table, lengths, scale=scale,
-                                  q_pos=q_pos, widths=width_d)
+                                  q_pos=q_pos, widths=width_d,
+                                  waves=ops.split_waves(pool.fmt, heads, length, batch, q.device))
         return out.to(dtype)
