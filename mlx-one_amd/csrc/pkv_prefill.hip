@@ -335,120 +335,20 @@ __global__ __launch_bounds__(64 * kMaxPrefillWaves) void prefill_kernel(const At
     return;
   }
 
-  // ---- the wave's query rows: row = ROWS*rblk + 16*RB*wv + 16*rb + col
+  // ---- the wave's query rows: row = ROWS*rblk + 16*RB*wv + 16*rb + col, and
+  // how far each sees.  The span comes before the queries themselves: the
+  // first stage's tiles are then requested before the query operands are
+  // loaded and converted, and both wait once (three f16 prompts of up to 1,000
+  // tokens: 60.4 -> 58.7 us; long spans within noise).
   int lim[RB];
-  QT qv[RB][KB];
-  // The query operand is the query itself; scale*log2(e) is applied to the
-  // f32 scores, never rounded into the operand.
-  const float rsc = a.scale_log2;
 #pragma unroll
   for (int rb = 0; rb < RB; ++rb) {
     const int row = rblk * ROWS + wv * 16 * RB + rb * 16 + col;
-    const bool valid = row < a.rows;
-    const int rowv = valid ? row : 0;  // rows past the block load row 0, zeroed below
-    const int qi = rowv / a.gqa, h = kh * a.gqa + rowv % a.gqa;
-    const bool live = valid && qi < width;
+    const int qi = (row < a.rows ? row : 0) / a.gqa;
+    const bool live = row < a.rows && qi < width;
     const int pos = a.q_pos ? a.q_pos[(int64_t)b * a.nq + qi] : L - width + qi;
     lim[rb] = live ? min(pos, L - 1) : -1;
-    const uint16_t *qrow = a.q + (((int64_t)b * a.heads + h) * a.nq + qi) * g.dim;
-#pragma unroll
-    for (int kb = 0; kb < KB; ++kb) {
-      const int d0 = 32 * kb + 8 * jj;
-      uint16_t e8[8];
-      if ((g.dim & 7) == 0) {
-        const u4 x = *(const u4 *)(qrow + (d0 < g.dim ? d0 : 0));
-        e8[0] = x.x & 0xFFFF; e8[1] = x.x >> 16; e8[2] = x.y & 0xFFFF; e8[3] = x.y >> 16;
-        e8[4] = x.z & 0xFFFF; e8[5] = x.z >> 16; e8[6] = x.w & 0xFFFF; e8[7] = x.w >> 16;
-      } else {
-#pragma unroll
-        for (int e = 0; e < 8; ++e) e8[e] = qrow[d0 + e < g.dim ? d0 + e : 0];
-      }
-#pragma unroll
-      for (int e = 0; e < 8; ++e)
-        if (!valid || d0 + e >= g.dim) e8[e] = 0;
-      qv[rb][kb] = __builtin_bit_cast(QT, u4{e8[0] | ((uint32_t)e8[1] << 16), e8[2] | ((uint32_t)e8[3] << 16),
-                                             e8[4] | ((uint32_t)e8[5] << 16), e8[6] | ((uint32_t)e8[7] << 16)});
-    }
   }
-
-  // Exact scores (quantized pages): per row block the B operand of the bias
-  // MFMA, the row's group sums of q times scale*log2(e), Q_g, in parts (the
-  // lane holds slots 4jj..4jj+3).  bf16 parts carry any magnitude.  f16
-  // parts (four or more groups) hold |Q_g| < 2^15: a row whose largest |Q_g|
-  // reaches it has its Q_g scaled by 2^-e, the MFMA then adds the bias term
-  // scaled by 2^-e to an accumulator scaled the same way, and the result is
-  // scaled back by 2^e; a wave holding such a row takes that general form of
-  // the final step (`wide`, a uniform branch).
-  BT qop[QUANT ? RB : 1];
-  float dn[QUANT ? RB : 1], ue[QUANT ? RB : 1];
-  bool wide_lane = false;
-  if constexpr (QUANT) {
-#pragma unroll
-    for (int rb = 0; rb < RB; ++rb) {
-      float qs[NG];
-#pragma unroll
-      for (int gi = 0; gi < NG; ++gi) qs[gi] = 0.0f;
-#pragma unroll
-      for (int kb = 0; kb < KB; ++kb) {
-        float t = 0.0f;
-#pragma unroll
-        for (int e = 0; e < 8; ++e) t += (float)qv[rb][kb][e];
-        qs[(32 * kb) / G] += t;
-      }
-#pragma unroll
-      for (int gi = 0; gi < NG; ++gi) {
-        qs[gi] += __shfl_xor(qs[gi], 16, 64);
-        qs[gi] += __shfl_xor(qs[gi], 32, 64);
-        qs[gi] *= rsc;
-      }
-      BT op = {0, 0, 0, 0};
-      auto place = [&](int k, auto v) __attribute__((always_inline)) {
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-          if ((k & 3) == i) op[i] = (k >> 2) == jj ? v : op[i];
-      };
-      if constexpr (BF16_BIAS) {
-        dn[rb] = ue[rb] = 1.0f;
-#pragma unroll
-        for (int gi = 0; gi < NG; ++gi) {
-          // three bf16 parts (24 bits): hi, mid, lo; each remainder is exact in f32
-          const uint16_t hi = f32_to_bf16_bits(qs[gi]);
-          const float r1 = qs[gi] - __uint_as_float((uint32_t)hi << 16);
-          const uint16_t mid = f32_to_bf16_bits(r1);
-          const uint16_t lo = f32_to_bf16_bits(r1 - __uint_as_float((uint32_t)mid << 16));
-          const short part[3] = {(short)hi, (short)mid, (short)lo};
-#pragma unroll
-          for (int pt = 0; pt < SPG; ++pt) place(gi * SPG + pt, part[pt % 3]);
-        }
-      } else {
-        float qmax = 0.0f;
-#pragma unroll
-        for (int gi = 0; gi < NG; ++gi) qmax = fmaxf(qmax, fabsf(qs[gi]));
-        int e = 0;
-        if (qmax >= 32768.0f && qmax < INFINITY) {
-          int ex;
-          frexpf(qmax, &ex);  // qmax in [2^(ex-1), 2^ex): qmax * 2^(15-ex) < 2^15
-          e = ex - 15;
-        }
-        dn[rb] = ldexpf(1.0f, -e);
-        ue[rb] = ldexpf(1.0f, e);
-        wide_lane |= e != 0;
-#pragma unroll
-        for (int gi = 0; gi < NG; ++gi) {
-          const float x = qs[gi] * dn[rb];
-          const _Float16 hi = (_Float16)x;
-          const float r1 = x - (float)hi;
-          const _Float16 mid = (_Float16)r1;
-          const _Float16 lo = (_Float16)(r1 - (float)mid);
-          const _Float16 part[3] = {hi, mid, lo};
-#pragma unroll
-          for (int pt = 0; pt < SPG; ++pt) place(gi * SPG + pt, part[pt]);
-        }
-      }
-      qop[rb] = op;
-    }
-  }
-  const bool wide = QUANT && !BF16_BIAS && __any(wide_lane);
 
   // ---- the block's visible span: tokens up to the largest limit; tiles
   // below the smallest live limit are seen whole by every live row
@@ -580,6 +480,119 @@ __global__ __launch_bounds__(64 * kMaxPrefillWaves) void prefill_kernel(const At
         load_meta<C>(rvm, head + g.vmeta_offset + (int64_t)((tip * PKV_TILE + 4 * jj) * NG) * 4);
     }
   };
+
+  if (nstages > 0) fetch(0);
+
+  // ---- the query operands
+  QT qv[RB][KB];
+  // The query operand is the query itself; scale*log2(e) is applied to the
+  // f32 scores, never rounded into the operand.
+  const float rsc = a.scale_log2;
+#pragma unroll
+  for (int rb = 0; rb < RB; ++rb) {
+    const int row = rblk * ROWS + wv * 16 * RB + rb * 16 + col;
+    const bool valid = row < a.rows;
+    const int rowv = valid ? row : 0;  // rows past the block load row 0, zeroed below
+    const int qi = rowv / a.gqa, h = kh * a.gqa + rowv % a.gqa;
+    const uint16_t *qrow = a.q + (((int64_t)b * a.heads + h) * a.nq + qi) * g.dim;
+#pragma unroll
+    for (int kb = 0; kb < KB; ++kb) {
+      const int d0 = 32 * kb + 8 * jj;
+      uint16_t e8[8];
+      if ((g.dim & 7) == 0) {
+        const u4 x = *(const u4 *)(qrow + (d0 < g.dim ? d0 : 0));
+        e8[0] = x.x & 0xFFFF; e8[1] = x.x >> 16; e8[2] = x.y & 0xFFFF; e8[3] = x.y >> 16;
+        e8[4] = x.z & 0xFFFF; e8[5] = x.z >> 16; e8[6] = x.w & 0xFFFF; e8[7] = x.w >> 16;
+      } else {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) e8[e] = qrow[d0 + e < g.dim ? d0 + e : 0];
+      }
+#pragma unroll
+      for (int e = 0; e < 8; ++e)
+        if (!valid || d0 + e >= g.dim) e8[e] = 0;
+      qv[rb][kb] = __builtin_bit_cast(QT, u4{e8[0] | ((uint32_t)e8[1] << 16), e8[2] | ((uint32_t)e8[3] << 16),
+                                             e8[4] | ((uint32_t)e8[5] << 16), e8[6] | ((uint32_t)e8[7] << 16)});
+    }
+  }
+
+  // Exact scores (quantized pages): per row block the B operand of the bias
+  // MFMA, the row's group sums of q times scale*log2(e), Q_g, in parts (the
+  // lane holds slots 4jj..4jj+3).  bf16 parts carry any magnitude.  f16
+  // parts (four or more groups) hold |Q_g| < 2^15: a row whose largest |Q_g|
+  // reaches it has its Q_g scaled by 2^-e, the MFMA then adds the bias term
+  // scaled by 2^-e to an accumulator scaled the same way, and the result is
+  // scaled back by 2^e; a wave holding such a row takes that general form of
+  // the final step (`wide`, a uniform branch).
+  BT qop[QUANT ? RB : 1];
+  float dn[QUANT ? RB : 1], ue[QUANT ? RB : 1];
+  bool wide_lane = false;
+  if constexpr (QUANT) {
+#pragma unroll
+    for (int rb = 0; rb < RB; ++rb) {
+      float qs[NG];
+#pragma unroll
+      for (int gi = 0; gi < NG; ++gi) qs[gi] = 0.0f;
+#pragma unroll
+      for (int kb = 0; kb < KB; ++kb) {
+        float t = 0.0f;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) t += (float)qv[rb][kb][e];
+        qs[(32 * kb) / G] += t;
+      }
+#pragma unroll
+      for (int gi = 0; gi < NG; ++gi) {
+        qs[gi] += __shfl_xor(qs[gi], 16, 64);
+        qs[gi] += __shfl_xor(qs[gi], 32, 64);
+        qs[gi] *= rsc;
+      }
+      BT op = {0, 0, 0, 0};
+      auto place = [&](int k, auto v) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          if ((k & 3) == i) op[i] = (k >> 2) == jj ? v : op[i];
+      };
+      if constexpr (BF16_BIAS) {
+        dn[rb] = ue[rb] = 1.0f;
+#pragma unroll
+        for (int gi = 0; gi < NG; ++gi) {
+          // three bf16 parts (24 bits): hi, mid, lo; each remainder is exact in f32
+          const uint16_t hi = f32_to_bf16_bits(qs[gi]);
+          const float r1 = qs[gi] - __uint_as_float((uint32_t)hi << 16);
+          const uint16_t mid = f32_to_bf16_bits(r1);
+          const uint16_t lo = f32_to_bf16_bits(r1 - __uint_as_float((uint32_t)mid << 16));
+          const short part[3] = {(short)hi, (short)mid, (short)lo};
+#pragma unroll
+          for (int pt = 0; pt < SPG; ++pt) place(gi * SPG + pt, part[pt % 3]);
+        }
+      } else {
+        float qmax = 0.0f;
+#pragma unroll
+        for (int gi = 0; gi < NG; ++gi) qmax = fmaxf(qmax, fabsf(qs[gi]));
+        int e = 0;
+        if (qmax >= 32768.0f && qmax < INFINITY) {
+          int ex;
+          frexpf(qmax, &ex);  // qmax in [2^(ex-1), 2^ex): qmax * 2^(15-ex) < 2^15
+          e = ex - 15;
+        }
+        dn[rb] = ldexpf(1.0f, -e);
+        ue[rb] = ldexpf(1.0f, e);
+        wide_lane |= e != 0;
+#pragma unroll
+        for (int gi = 0; gi < NG; ++gi) {
+          const float x = qs[gi] * dn[rb];
+          const _Float16 hi = (_Float16)x;
+          const float r1 = x - (float)hi;
+          const _Float16 mid = (_Float16)r1;
+          const _Float16 lo = (_Float16)(r1 - (float)mid);
+          const _Float16 part[3] = {hi, mid, lo};
+#pragma unroll
+          for (int pt = 0; pt < SPG; ++pt) place(gi * SPG + pt, part[pt]);
+        }
+      }
+      qop[rb] = op;
+    }
+  }
+  const bool wide = QUANT && !BF16_BIAS && __any(wide_lane);
 
   // ---- convert the raw tile into slot wv of a stage image (K half, then V
   // half: each is scheduled against one step's MFMAs)
@@ -910,7 +923,6 @@ __global__ __launch_bounds__(64 * kMaxPrefillWaves) void prefill_kernel(const At
   // invalid (zeros, fully masked), and the last stage converts the absent
   // tile past the span into the image nobody reads again.
   if (nstages > 0) {
-    fetch(0);
     convert(0, true);
     convert(0, false);
     if (nstages > 1) fetch(1);
