@@ -186,7 +186,7 @@ int attention_group_waves();
 int attention_slots(const Geo &g, int rows);
 int attention_group_lead();
 // Whether the split-K decode kernel serves this many rows per KV head (else
-// launch_prefill does, with no workspace and no merge).
+// launch_prefill does).
 bool decode_serves(const Geo &g, int rows);
 // Whether the decode kernel fuses the single-token append for this layout and
 // row count (at most 8 rows per KV head).
