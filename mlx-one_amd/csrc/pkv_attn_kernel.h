@@ -492,7 +492,10 @@ __attribute__((amdgpu_waves_per_eu(min_waves_per_simd(BITS, DP, G, RB, SLOTS))))
   int app_pid = -1;
   auto append_fetch = [&](int pb, int pkh, int pos) __attribute__((always_inline)) {
     if constexpr (APPEND) {
-      app_pid = a.table[(int64_t)pb * a.max_pages + pos / g.page];
+      // (a position past the block table has no page: the token is dropped, as
+      // the append kernels drop it)
+      const int slot = pos / g.page;
+      app_pid = slot < a.max_pages ? a.table[(int64_t)pb * a.max_pages + slot] : -1;
       const int64_t row = ((int64_t)pb * hk + pkh) * g.dim;
 #pragma unroll
       for (int side = 0; side < 2; ++side) {
