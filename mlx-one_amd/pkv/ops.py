@@ -173,13 +173,14 @@ _PLANS = {}
 _MAX_PLANS = 4096
 
 
-def _plan(fmt, heads, nq, batch, device, wide=False):
-    """The default waves of a call and the workspace it runs best with."""
+def _plan(fmt, heads, nq, batch, device):
+    """The default waves of a call and the workspace it runs best with, the same
+    whichever entry point asks first."""
     key = (fmt, heads, nq, batch, device)
     plan = _PLANS.get(key)
     if plan is None:
         waves = default_waves(fmt, heads, decode_queries(fmt, heads, nq) or nq, batch)
-        plan = (waves, _workspace_need(fmt, heads, nq, batch, waves, wide))
+        plan = (waves, _workspace_need(fmt, heads, nq, batch, waves))
         if len(_PLANS) >= _MAX_PLANS:
             _PLANS.clear()
         _PLANS[key] = plan
@@ -191,11 +192,17 @@ def split_waves(fmt, heads, nq, batch, device):
     equal split over them, whatever its block table's width -- the arenas' calls
     give the same bits from host tables (as wide as the batch) and from the
     device's (as wide as ``max_tokens``)."""
-    return _plan(fmt, heads, nq, batch, device, decode_queries(fmt, heads, nq) != nq)[0]
+    return _plan(fmt, heads, nq, batch, device)[0]
 
 
-def _workspace_need(fmt, heads, nq, batch, waves, wide):
-    if wide:
+def is_wide(fmt, heads, nq):
+    """Whether the prefill kernel serves a call's query blocks (more rows per KV
+    head than the decode kernel takes)."""
+    return decode_queries(fmt, heads, nq) != nq
+
+
+def _workspace_need(fmt, heads, nq, batch, waves):
+    if is_wide(fmt, heads, nq):
         need = int(nat.load().pkv_attention_batch_workspace_bytes(fmt.c_layout, heads, nq, batch,
                                                                   waves))
     else:
@@ -245,13 +252,13 @@ def paged_attention(fmt: PageFormat, pool, queries, block_table, seq_lens, *, sc
     lens = _i32(seq_lens, device)
     # a wide call has room for split prefill spans too, in the stream's own
     # memory: wide calls on other streams or threads may overlap this one
-    wide = decode_queries(fmt, heads, nq) != nq
+    wide = is_wide(fmt, heads, nq)
     if waves <= 0:
-        waves, need = _plan(fmt, heads, nq, batch, device, wide)
+        waves, need = _plan(fmt, heads, nq, batch, device)
         if not wide:
             waves = 0  # the library's choice, within the workspace of its default waves
     else:
-        need = _workspace_need(fmt, heads, nq, batch, waves, wide)
+        need = _workspace_need(fmt, heads, nq, batch, waves)
     if workspace is None:
         workspace = (torch.empty(max(need, 256), dtype=torch.uint8, device=device) if wide
                      else attention_workspace(device, need))
@@ -300,7 +307,7 @@ def append_paged_attention(fmt: PageFormat, pool, keys, values, queries, block_t
     if waves <= 0:
         waves, need = 0, _plan(fmt, heads, 1, batch, device)[1]
     else:
-        need = _workspace_need(fmt, heads, 1, batch, waves, False)
+        need = _workspace_need(fmt, heads, 1, batch, waves)
     if workspace is None:
         workspace = attention_workspace(device, need)
     elif workspace.device != device or workspace.dtype != torch.uint8 or \
