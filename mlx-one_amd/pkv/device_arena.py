@@ -338,12 +338,13 @@ class DeviceRunner:
         slots_d = torch.tensor([int(s) for s in slots], dtype=torch.int32, device=device)
         widths_d = torch.ones_like(slots_d)
         count = int(slots_d.numel())
-        # the graph's split-K partials live in a workspace of its own, sized
-        # for the waves fixed at capture and held by the CapturedStep
+        # the graph's split-K partials live in a workspace of its own, sized as an
+        # eager call's (so both run the same split) for the waves fixed at
+        # capture, and held by the CapturedStep
         spec = self.model.spec
         waves = ops.default_waves(arena.fmt, spec.query_heads, 1, count)
-        workspace = torch.empty(max(256, ops.workspace_bytes(arena.fmt, spec.query_heads, 1,
-                                                             waves)),
+        workspace = torch.empty(max(256, ops.call_workspace_bytes(arena.fmt, spec.query_heads, 1,
+                                                                  count, waves)),
                                 dtype=torch.uint8, device=device)
         if warm:
             res = arena.reserve(slots_d, widths_d)

@@ -180,7 +180,7 @@ def _plan(fmt, heads, nq, batch, device):
     plan = _PLANS.get(key)
     if plan is None:
         waves = default_waves(fmt, heads, decode_queries(fmt, heads, nq) or nq, batch)
-        plan = (waves, _workspace_need(fmt, heads, nq, batch, waves))
+        plan = (waves, call_workspace_bytes(fmt, heads, nq, batch, waves))
         if len(_PLANS) >= _MAX_PLANS:
             _PLANS.clear()
         _PLANS[key] = plan
@@ -201,7 +201,10 @@ def is_wide(fmt, heads, nq):
     return decode_queries(fmt, heads, nq) != nq
 
 
-def _workspace_need(fmt, heads, nq, batch, waves):
+def call_workspace_bytes(fmt, heads, nq, batch, waves):
+    """Workspace with which a call of ``batch`` sequences runs best (and which
+    the calls below take when given none): ``workspace_bytes``, and for a wide
+    call the partials of cut prefill spans as well."""
     if is_wide(fmt, heads, nq):
         need = int(nat.load().pkv_attention_batch_workspace_bytes(fmt.c_layout, heads, nq, batch,
                                                                   waves))
@@ -227,6 +230,16 @@ def attention_workspace(device, nbytes):
     return ws
 
 
+def _own_workspace(fmt, heads, nq, device, nbytes):
+    """The workspace of a call that was given none: the device's shared one, or
+    for a wide call the stream's own memory of exactly that size -- wide calls
+    on other streams or threads may overlap it, and whether spans are cut (and
+    so the output's bits) must not depend on what grew the shared one."""
+    if is_wide(fmt, heads, nq):
+        return torch.empty(max(nbytes, 256), dtype=torch.uint8, device=device)
+    return attention_workspace(device, nbytes)
+
+
 def paged_attention(fmt: PageFormat, pool, queries, block_table, seq_lens, *, scale, q_pos=None,
                     widths=None, waves=0, workspace=None, out=None):
     """Attention of ``queries [B, H, Q, D]`` over the paged cache.
@@ -250,18 +263,14 @@ def paged_attention(fmt: PageFormat, pool, queries, block_table, seq_lens, *, sc
     device = queries.device
     table = _i32(block_table, device)
     lens = _i32(seq_lens, device)
-    # a wide call has room for split prefill spans too, in the stream's own
-    # memory: wide calls on other streams or threads may overlap this one
-    wide = is_wide(fmt, heads, nq)
     if waves <= 0:
         waves, need = _plan(fmt, heads, nq, batch, device)
-        if not wide:
+        if not is_wide(fmt, heads, nq):
             waves = 0  # the library's choice, within the workspace of its default waves
     else:
-        need = _workspace_need(fmt, heads, nq, batch, waves)
+        need = call_workspace_bytes(fmt, heads, nq, batch, waves)
     if workspace is None:
-        workspace = (torch.empty(max(need, 256), dtype=torch.uint8, device=device) if wide
-                     else attention_workspace(device, need))
+        workspace = _own_workspace(fmt, heads, nq, device, need)
     elif workspace.device != device or workspace.dtype != torch.uint8 or \
             not workspace.is_contiguous():
         raise ValueError("attention workspace must be a contiguous uint8 tensor on the "
@@ -307,9 +316,9 @@ def append_paged_attention(fmt: PageFormat, pool, keys, values, queries, block_t
     if waves <= 0:
         waves, need = 0, _plan(fmt, heads, 1, batch, device)[1]
     else:
-        need = _workspace_need(fmt, heads, 1, batch, waves)
+        need = call_workspace_bytes(fmt, heads, 1, batch, waves)
     if workspace is None:
-        workspace = attention_workspace(device, need)
+        workspace = _own_workspace(fmt, heads, 1, device, need)
     elif workspace.device != device or workspace.dtype != torch.uint8 or \
             not workspace.is_contiguous():
         raise ValueError("attention workspace must be a contiguous uint8 tensor on the "

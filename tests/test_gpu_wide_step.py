@@ -48,3 +48,60 @@ def test_bits_do_not_depend_on_the_order_of_calls(heads):
     _forget()
     again = fused(), attend()
     assert torch.equal(first[0], again[1]) and torch.equal(first[1], again[0])
+
+
+@pytest.mark.parametrize("heads", [40, 71])
+def test_bits_do_not_depend_on_the_shared_workspace(heads):
+    from pkv import ops
+
+    fused, _ = _case(heads)
+    _forget()
+    first = fused()
+    ops.attention_workspace(torch.device("cuda", 0), 64 << 20)
+    assert torch.equal(first, fused())
+
+
+@pytest.mark.parametrize("heads", [40, 71])
+def test_two_streams(heads):
+    """Steps on two streams at once give the bits they give alone, with a shared
+    workspace large enough for either's partials."""
+    from pkv import ops
+
+    steps = [_case(heads, seed, (6000, 2000 + seed))[0] for seed in (0, 1)]
+    ops.attention_workspace(torch.device("cuda", 0), 64 << 20)
+    want = [step() for step in steps]
+    streams = [torch.cuda.Stream() for _ in steps]
+    for s in streams:
+        s.wait_stream(torch.cuda.current_stream())
+    got = [[], []]
+    for _ in range(30):
+        for i, s in enumerate(streams):
+            with torch.cuda.stream(s):
+                got[i].append(steps[i]())
+    torch.cuda.synchronize()
+    for outs, w in zip(got, want):
+        assert all(torch.equal(out, w) for out in outs)
+
+
+def test_captured_step_equals_the_eager_one():
+    from pkv.device_arena import DevicePageArena, DeviceRunner
+    from pkv.layer import AttentionStack, ModelSpec
+    from pkv.ops import PageFormat
+
+    spec = ModelSpec(hidden=128, query_heads=40, kv_heads=1, head_dim=64, num_layers=2, dtype="bfloat16")
+    model = AttentionStack(spec, device="cuda", seed=3)
+    arena = DevicePageArena(PageFormat(1, 64, 16, 8, 64), 400, num_layers=2, max_slots=2, max_tokens=3000)
+    runner = DeviceRunner(model, arena)
+    slots = [arena.open_slot() for _ in range(2)]
+    gen = torch.Generator(device="cuda").manual_seed(1)
+    draw = lambda n: torch.randn((2, n, 128), generator=gen, device="cuda").to(torch.bfloat16)
+    runner.execute(slots, draw(2400), [2400, 1100])
+    step = runner.capture_decode(slots, draw(1))
+    for _ in range(3):
+        before = list(arena.lengths)
+        step.hidden.copy_(draw(1))
+        step.replay()
+        out = step.out.clone()
+        arena.truncate(slots, before)
+        eager = runner.execute(slots, step.hidden)
+        assert torch.equal(out, eager)
