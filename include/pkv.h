@@ -199,6 +199,10 @@ int pkv_paged_attention_noalloc(void *stream, const pkv_layout *layout, const vo
 #define PKV_DECODE_VALU 1
 int pkv_select_decode_kernel(int kind);
 
+/* Where the present choice stands (PKV_DECODE_*), for callers that keep sizes
+ * computed under it: valid while the library is loaded. */
+const int32_t *pkv_decode_kernel_choice(void);
+
 /*
  * Measurement aid, no counterpart in the reference: a plain streaming read of
  * whole pages (every KV head), page_ids[0..count) in order, split into equal

@@ -214,6 +214,8 @@ int pkv_select_decode_kernel(int kind) {
   return pkv::select_decode_kernel(kind);
 }
 
+const int32_t *pkv_decode_kernel_choice(void) { return pkv::decode_kernel_choice(); }
+
 int32_t pkv_attention_waves(const pkv_layout *layout, int32_t num_heads, int32_t num_queries) {
   pkv_geometry g;
   if (geometry(layout, &g) != PKV_OK) return -1;

@@ -561,9 +561,12 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void va
 
 // The decode kernel for at most 4 rows per KV head over quantized pages at
 // head_dim <= 128: attn_kernel (MFMA, the default) or valu_kernel.
-static std::atomic<int> g_decode_kernel{kDecodeMfma};
+static std::atomic<int32_t> g_decode_kernel{kDecodeMfma};
+static_assert(sizeof(g_decode_kernel) == sizeof(int32_t) && std::atomic<int32_t>::is_always_lock_free,
+              "read as a plain word by callers of decode_kernel_choice");
 
 int select_decode_kernel(int kind) { return g_decode_kernel.exchange(kind); }
+const int32_t *decode_kernel_choice() { return reinterpret_cast<const int32_t *>(&g_decode_kernel); }
 int decode_kernel() { return g_decode_kernel.load(); }
 
 static AttnKernel select_valu(const Geo &g) {

@@ -195,6 +195,7 @@ bool append_fusable(const Geo &g, int rows);
 // 128): process-wide; select returns the previous choice.
 constexpr int kDecodeMfma = 0, kDecodeValu = 1;
 int select_decode_kernel(int kind);
+const int32_t *decode_kernel_choice();  // where the choice stands
 int decode_kernel();
 
 }  // namespace pkv

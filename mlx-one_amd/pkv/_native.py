@@ -43,6 +43,7 @@ SIGNATURES = {
     "pkv_append_paged_attention": ([_c_p, _LP, _c_p, _i64, _c_p, _c_p, _c_p, _i32, _i32, _c_p,
                                     _i32, _c_p, _f32, _i32, _c_p, _i64, _c_p], ctypes.c_int),
     "pkv_select_decode_kernel": ([ctypes.c_int], ctypes.c_int),
+    "pkv_decode_kernel_choice": ([], _c_p),
     "pkv_attention_waves": ([_LP, _i32, _i32], _i32),
     "pkv_attention_default_waves": ([_LP, _i32, _i32, _i32], _i32),
     "pkv_attention_workspace_bytes": ([_LP, _i32, _i32, _i32], _i64),
@@ -101,6 +102,8 @@ def load(path=None):
         for name, (args, res) in SIGNATURES.items():
             fn = getattr(lib, name)
             fn.argtypes, fn.restype = args, res
+        # the library's own word, read without a call
+        lib.decode_kernel = ctypes.c_int32.from_address(lib.pkv_decode_kernel_choice())
         if path is None:
             _lib = lib
         return lib

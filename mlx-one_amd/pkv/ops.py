@@ -136,7 +136,6 @@ def select_decode_kernel(kind):
     if kind not in DECODE_KERNELS:
         raise ValueError(f"decode kernel must be one of {sorted(DECODE_KERNELS)}")
     previous = int(nat.load().pkv_select_decode_kernel(DECODE_KERNELS[kind]))
-    _PLANS.clear()
     if previous < 0:
         nat.check(previous, "select decode kernel")
     return {v: k for k, v in DECODE_KERNELS.items()}[previous]
@@ -166,21 +165,21 @@ def workspace_bytes(fmt: PageFormat, num_heads, num_queries, waves):
                                                           waves))
 
 
-# (waves, workspace bytes) of a call shape with default waves: a few integers
-# per format, heads, queries, batch and device, as the library computed them
-# (cleared when the decode kernel changes, and when it holds many shapes).
+# (waves, workspace bytes, wide) of a call shape with default waves: a few integers
+# per format, heads, queries, batch, device and decode kernel, as the library
+# computed them (cleared when it holds many shapes).
 _PLANS = {}
 _MAX_PLANS = 4096
 
 
 def _plan(fmt, heads, nq, batch, device):
-    """The default waves of a call and the workspace it runs best with, the same
-    whichever entry point asks first."""
-    key = (fmt, heads, nq, batch, device)
+    """The default waves of a call, the workspace it runs best with and whether
+    it is wide, the same whichever entry point asks first."""
+    key = (fmt, heads, nq, batch, device, nat.load().decode_kernel.value)
     plan = _PLANS.get(key)
     if plan is None:
         waves = default_waves(fmt, heads, decode_queries(fmt, heads, nq) or nq, batch)
-        plan = (waves, call_workspace_bytes(fmt, heads, nq, batch, waves))
+        plan = (waves, call_workspace_bytes(fmt, heads, nq, batch, waves), is_wide(fmt, heads, nq))
         if len(_PLANS) >= _MAX_PLANS:
             _PLANS.clear()
         _PLANS[key] = plan
@@ -230,14 +229,12 @@ def attention_workspace(device, nbytes):
     return ws
 
 
-def _own_workspace(fmt, heads, nq, device, nbytes):
-    """The workspace of a call that was given none: the device's shared one, or
-    for a wide call the stream's own memory of exactly that size -- wide calls
-    on other streams or threads may overlap it, and whether spans are cut (and
-    so the output's bits) must not depend on what grew the shared one."""
-    if is_wide(fmt, heads, nq):
-        return torch.empty(max(nbytes, 256), dtype=torch.uint8, device=device)
-    return attention_workspace(device, nbytes)
+def _wide_workspace(device, nbytes):
+    """The workspace of a wide call that was given none: the stream's own memory
+    of exactly that size -- wide calls on other streams or threads may overlap
+    it, and whether spans are cut (and so the output's bits) must not depend on
+    what grew the shared one."""
+    return torch.empty(max(nbytes, 256), dtype=torch.uint8, device=device)
 
 
 def paged_attention(fmt: PageFormat, pool, queries, block_table, seq_lens, *, scale, q_pos=None,
@@ -264,13 +261,13 @@ def paged_attention(fmt: PageFormat, pool, queries, block_table, seq_lens, *, sc
     table = _i32(block_table, device)
     lens = _i32(seq_lens, device)
     if waves <= 0:
-        waves, need = _plan(fmt, heads, nq, batch, device)
-        if not is_wide(fmt, heads, nq):
+        waves, need, wide = _plan(fmt, heads, nq, batch, device)
+        if not wide:
             waves = 0  # the library's choice, within the workspace of its default waves
     else:
-        need = call_workspace_bytes(fmt, heads, nq, batch, waves)
+        need, wide = call_workspace_bytes(fmt, heads, nq, batch, waves), is_wide(fmt, heads, nq)
     if workspace is None:
-        workspace = _own_workspace(fmt, heads, nq, device, need)
+        workspace = _wide_workspace(device, need) if wide else attention_workspace(device, need)
     elif workspace.device != device or workspace.dtype != torch.uint8 or \
             not workspace.is_contiguous():
         raise ValueError("attention workspace must be a contiguous uint8 tensor on the "
@@ -314,11 +311,11 @@ def append_paged_attention(fmt: PageFormat, pool, keys, values, queries, block_t
     table = _i32(block_table, device)
     lens = _i32(seq_lens, device)
     if waves <= 0:
-        waves, need = 0, _plan(fmt, heads, 1, batch, device)[1]
+        waves, (_, need, wide) = 0, _plan(fmt, heads, 1, batch, device)
     else:
-        need = call_workspace_bytes(fmt, heads, 1, batch, waves)
+        need, wide = call_workspace_bytes(fmt, heads, 1, batch, waves), is_wide(fmt, heads, 1)
     if workspace is None:
-        workspace = _own_workspace(fmt, heads, 1, device, need)
+        workspace = _wide_workspace(device, need) if wide else attention_workspace(device, need)
     elif workspace.device != device or workspace.dtype != torch.uint8 or \
             not workspace.is_contiguous():
         raise ValueError("attention workspace must be a contiguous uint8 tensor on the "

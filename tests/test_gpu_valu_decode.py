@@ -225,3 +225,35 @@ def test_select_decode_kernel_rejects_unknown_kinds():
     lib = _native.load()
     assert lib.pkv_select_decode_kernel(7) == _native.PKV_INVALID_ARGUMENT
     assert ops.select_decode_kernel("valu") == "valu"
+
+
+def test_choice_made_through_the_library_reaches_the_next_call():
+    """The decode kernel switched past ``ops`` (any caller of the library may):
+    workspaces sized for one kernel's waves are not passed to the other, and the
+    bits are those of the kernel chosen when the call launches."""
+    from pkv import _native, ops, workloads
+
+    lib = _native.load()
+    w = workloads.get("c2", batch=2, lengths=(3000, 2200), num_queries=1, append_tokens=1,
+                      shared_prefix_pages=0)
+    inst = workloads.generate(w)
+    fmt = _fmt(w)
+    pool, table, lengths = fill_pages(fmt, inst, chunk=512)
+    q = to_torch(inst.queries, fmt.dtype)
+
+    def call():
+        ops._WORKSPACES.clear()
+        return ops.paged_attention(fmt, pool, q, table, lengths, scale=scale_of(w.head_dim))
+
+    want = []
+    for kind in (0, 1):
+        lib.pkv_select_decode_kernel(kind)
+        assert lib.decode_kernel.value == kind
+        ops._PLANS.clear()
+        want.append(call())
+    for order in ((0, 1), (1, 0)):
+        ops._PLANS.clear()
+        for kind in order:
+            lib.pkv_select_decode_kernel(kind)
+            assert torch.equal(call(), want[kind])
+    lib.pkv_select_decode_kernel(1)
