@@ -210,27 +210,26 @@ __device__ __forceinline__ PrefillGrid prefill_grid(const AttnArgs &a, int lane)
   return p;
 }
 
-// Workgroup -> (segment, row block, piece).  Blocks of one segment read the same
-// pages: they go to one XCD (workgroups are dealt to the 8 XCDs round-robin),
-// so its span is fetched into one L2.  With a multiple of 8 segments XCD x
-// runs segments x, x + 8, ... (heavy segments that sit together in the batch
-// still spread over every XCD), the longest spans of all of them (a causal
-// chunk's last row blocks) first, so that the grid does not end on them: three
-// f16 prompts of 1,000 tokens (384 blocks of 1 to 8 stages on 256 CUs)
-// 78 -> 62 us.  Otherwise each XCD takes an eighth of the blocks, in segment order.
+// Workgroup -> (segment, row block, piece): segments vary fastest, then a span's
+// pieces, the row blocks from the last (a causal chunk's longest spans) to the
+// first, so that the grid does not end on its longest spans: three f16 prompts
+// of 1,000 tokens (384 blocks of 1 to 8 stages on 256 CUs) 78 -> 62 us.
+// Workgroups are dealt to the 8 XCDs round-robin, so with a multiple of 8
+// segments XCD x runs segments x, x + 8, ... and fetches each span into one L2;
+// heavy segments that sit together in the batch still spread over every XCD.
+// Two or four segments of whole spans go one after the other instead, each over
+// every XCD: an XCD that keeps to one of them has more rounds of work than
+// another where the sequences differ (two prompts of 1,200 and 980 tokens behind
+// 3,000 to 3,750, 2 KV heads of 256 bf16 dims, 7 heads each: 408 us; 568 with the
+// segments side by side, 619 with an eighth of the blocks to each XCD).
 __device__ __forceinline__ void prefill_item(const PrefillGrid &p, int bid, int &seg, int &rblk, int &piece) {
-  const int x = bid & 7;
-  int k = bid >> 3;
-  if ((p.nseg & 7) == 0) {
-    const int spx = p.nseg >> 3;
-    seg = x + 8 * (k % spx);
-    k /= spx;
+  int k;
+  if (p.split == 1 && (p.nseg == 2 || p.nseg == 4)) {
+    seg = bid / p.nblk;
+    k = bid - seg * p.nblk;
   } else {
-    const int total = p.nseg * p.nblk * p.split;
-    k += x * (total >> 3) + min(x, total & 7);
-    const int per = p.nblk * p.split;
-    seg = k / per;
-    k -= seg * per;
+    k = bid / p.nseg;
+    seg = bid - k * p.nseg;
   }
   piece = k % p.split;
   rblk = p.nblk - 1 - k / p.split;
