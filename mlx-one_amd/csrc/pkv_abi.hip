@@ -78,26 +78,29 @@ WorkspaceParts workspace_parts(const pkv_geometry &g, int64_t rows, int64_t wave
   return w;
 }
 
-// Partials of split prefill spans (prefill_split) for a wide call of `batch`
-// sequences: [pieces per row block: int32][ml][acc] with `blocks` pieces of one
-// workgroup's rows each; no blocks where no span can be split.  `share`: a
-// mixed batch, whose live sequences the host does not know (one or more).
+// Partials of cut prefill spans (prefill_longest) for a wide call of `batch`
+// sequences of at most `tokens` tokens: [pieces per row block: int32][ml][acc]
+// with `blocks` pieces of one workgroup's rows each; none where no span can be
+// cut.  `share`: a mixed batch, whose live sequences the host does not know (one
+// or more).
 struct PrefillParts {
-  int cus;  // 0: no split
+  int cus, units;  // cus 0: no span is cut
   int64_t blocks, ml, acc, total;
 };
 
-PrefillParts prefill_parts(const pkv_geometry &g, int64_t rows, int64_t batch, bool share) {
-  PrefillParts p{0, 0, 0, 0, 0};
+PrefillParts prefill_parts(const pkv_geometry &g, int64_t rows, int64_t batch, bool share, int64_t tokens) {
+  PrefillParts p{0, 0, 0, 0, 0, 0};
   const pkv::Geo geo = pkv::to_geo(g);
   const int cus = pkv::device_cus();
-  const int64_t per_seq = (int64_t)g.hk * pkv::prefill_blocks(geo, (int)rows);
-  const int64_t least = share ? per_seq : per_seq * batch;
-  if (cus <= 0 || pkv::prefill_split(least, cus) < 2) return p;
+  const int units = (int)std::min<int64_t>((tokens + pkv::kPrefillUnit - 1) / pkv::kPrefillUnit, 1 << 24);
+  const pkv::PrefillCut cut =
+      pkv::prefill_cut((int64_t)g.hk * pkv::prefill_blocks(geo, (int)rows), batch, share, units, cus);
+  if (cus <= 0 || cut.items == 0) return p;
   p.cus = cus;
-  p.blocks = share ? 2 * (int64_t)cus : least * pkv::prefill_split(least, cus);
+  p.units = units;
+  p.blocks = cut.parts;
   const int64_t block_rows = pkv::prefill_block_rows(geo);
-  p.ml = align256(p.blocks * 4);
+  p.ml = align256(cut.items * 4);
   p.acc = p.ml + align256(p.blocks * block_rows * 2 * 4);
   p.total = p.acc + align256(p.blocks * block_rows * g.dp * 4);
   return p;
@@ -284,8 +287,9 @@ int64_t pkv_attention_batch_workspace_bytes(const pkv_layout *layout, int32_t nu
   int64_t parts = 0;
   if (lo >= 1) parts += align256(workspace_parts(g, (int64_t)lo * gqa, waves, 0).total);
   if (hi > lo) parts += align256(workspace_parts(g, (int64_t)hi * gqa, waves, 0).total);
-  const int64_t mixed = parts + prefill_parts(g, rows, batch, hi >= 1).total;
-  return std::max(need, std::max(mixed, prefill_parts(g, rows, batch, false).total));
+  // (for block tables of any width)
+  const int64_t mixed = parts + prefill_parts(g, rows, batch, hi >= 1, INT64_MAX / 2).total;
+  return std::max(need, std::max(mixed, prefill_parts(g, rows, batch, false, INT64_MAX / 2).total));
 }
 
 }  // extern "C"
@@ -383,19 +387,20 @@ int paged_attention_impl(void *stream, const pkv_layout *layout, const void *poo
   // where its row blocks leave CUs idle.  (A workspace sized for the decode parts
   // alone, and the library's own scratch, run the parts and their merges one
   // after the other over one region, and no span is cut.)
-  PrefillParts pre{0, 0, 0, 0, 0};
+  PrefillParts pre{0, 0, 0, 0, 0, 0};
   bool together = false;
   int64_t part_base[2] = {0, 0};
   if (wide && !fit_waves && workspace) {
-    pre = prefill_parts(geo, rows, batch, nparts > 0);
+    pre = prefill_parts(geo, rows, batch, nparts > 0, (int64_t)max_pages * geo.page);
     int64_t total = pre.total;
     for (int i = 0; i < nparts; ++i) {
       part_base[i] = total;
       total += align256(part[i].ws.total);
     }
-    together = workspace_bytes >= total && total > 0;
+    // (one part and nothing cut: its own merge is the one launch)
+    together = workspace_bytes >= total && (pre.cus > 0 || nparts > 1);
     if (!together) {
-      pre = PrefillParts{0, 0, 0, 0, 0};
+      pre = PrefillParts{0, 0, 0, 0, 0, 0};
       part_base[0] = part_base[1] = 0;
     }
   }
@@ -454,6 +459,7 @@ int paged_attention_impl(void *stream, const pkv_layout *layout, const void *poo
     a.part_acc = nullptr;
     if (pre.cus > 0) {
       a.pre_cus = pre.cus;
+      a.pre_units = pre.units;
       a.pre_cnt = (int32_t *)workspace;
       a.pre_ml = (float *)((char *)workspace + pre.ml);
       a.pre_acc = (float *)((char *)workspace + pre.acc);

@@ -63,10 +63,11 @@ struct AttnArgs {
   // the pool, writable) by the wave that attends the sequence's last tile.
   uint8_t *wpool = nullptr;
   const uint16_t *new_k = nullptr, *new_v = nullptr;
-  // Prefill kernel: the CUs to fill (0: no split) and the partials of spans cut
-  // into pieces (prefill_split): pieces per row block, then per piece the rows'
-  // (m, l) [block*S + piece][rows per block][2] and O^T as its lanes hold it.
-  int pre_cus = 0;
+  // Prefill kernel: the CUs to fill (0: no span is cut), the units of the longest
+  // span the block table can hold, and the partials of spans cut into pieces
+  // (prefill_longest): pieces per row block, then per piece the rows' (m, l)
+  // [block*S + piece][rows per block][2] and O^T as its lanes hold it.
+  int pre_cus = 0, pre_units = 0;
   int32_t *pre_cnt = nullptr;
   float *pre_ml = nullptr, *pre_acc = nullptr;
 };
@@ -80,17 +81,72 @@ struct MergeArgs {
   uint16_t *out;
 };
 
-// Pieces the span of each row block is cut into when `blocks` prefill workgroups
-// (one per CU: LDS) would leave CUs idle: as many as fill the CUs once, or
-// twice where that is over 10% shorter (three pieces in two rounds of a grid
-// between half and two thirds of the CUs).  At most two pieces per CU (the
-// partials' space) and kMaxPrefillSplit per span.
+// A sequence of `units` units of 128 tokens in a prefill grid of `blocks` row
+// blocks (one workgroup per CU each: LDS) that would leave CUs idle: the longest
+// piece its row blocks' spans are cut into, in units (all of them: whole spans).
+// A unit takes about 4.2 us (head_dim 128), a piece a step of the merge, which
+// walks them in order, and its partials, so the best number of pieces grows as
+// the root of the units: sqrt(2 * units) is within 4% of it for 8 to 32 blocks of
+// 6 to 64 units at head_dim 64, 128 and 256, and past 32 blocks the CUs bound it
+// (8 blocks of 64 units, 8-bit pages: 278 us whole, 89 in 4 pieces, 62 in 11, 77
+// in 32).  Sequences of less than 4 units stay whole, and of a few more where
+// many blocks would write partials (64 blocks of 4: 32.2 us, 35.0 in two pieces;
+// 96 of 6: 41.0 and 37.9; 128 of 6: 41.5 and 40.7, of 8: 49.3 and 45.3).
+// More pieces than CUs, in two rounds, where their shorter rounds save 6 units,
+// the second start-up and its partials (160 blocks, three pieces: 12 units 67 us
+// whole, 78 cut).
 constexpr int kMaxPrefillSplit = 32;
-__host__ __device__ inline int prefill_split(int64_t blocks, int cus) {
-  if (blocks < 1 || blocks > cus) return 1;
-  const uint32_t once = (uint32_t)cus / (uint32_t)blocks, twice = 2 * (uint32_t)cus / (uint32_t)blocks;
-  const uint32_t s = 9 * twice > 20 * once ? twice : once;
-  return s < kMaxPrefillSplit ? (int)s : kMaxPrefillSplit;
+constexpr int kPrefillUnit = 128;  // tokens: the largest page, one or two stages
+struct PrefillRounds {
+  int once, twice;  // pieces per span that fill the CUs once and twice (0: no span is cut)
+  __host__ __device__ PrefillRounds(int64_t blocks, int units, int cus) {
+    const bool whole = units < 4 || blocks < 1 || blocks > cus || blocks > 32 * ((int64_t)units - 3);
+    once = whole ? 0 : cus / (int)blocks;
+    twice = whole ? 0 : 2 * cus / (int)blocks;
+    if (twice > kMaxPrefillSplit) twice = kMaxPrefillSplit;
+    if ((int64_t)units * (twice - 2 * once) <= (int64_t)6 * once * twice) twice = 0;  // not worth it
+    // the root of the units, at most once
+    int p = 1;
+    while (p < once && p < kMaxPrefillSplit && (p + 1) * (p + 1) <= 2 * units) ++p;
+    once = p;
+  }
+};
+__host__ __device__ inline int prefill_longest(int units, int64_t blocks, int cus) {
+  const PrefillRounds r(blocks, units, cus);
+  const int pieces = r.twice > 0 ? r.twice : r.once;
+  return (units + pieces - 1) / pieces;
+}
+
+// The most pieces a span is cut into there, in sequences of up to `units` units;
+// with `zeros` (a mixed batch's dead rows to be written by the grid as well) at
+// least as many workgroups per row block as fill the CUs.
+__host__ __device__ inline int prefill_split(int units, int64_t blocks, int cus, bool zeros) {
+  const PrefillRounds r(blocks, units, cus);
+  int p = r.twice > r.once ? r.twice : r.once;
+  if (zeros && blocks > 0 && cus / (int)blocks > p) p = cus / (int)blocks;
+  return p < kMaxPrefillSplit ? p : kMaxPrefillSplit;
+}
+
+// What a wide call's prefill grid may need where it has CUs to fill; with `share`
+// (a mixed batch, whose live sequences only the device knows) over any number of
+// live sequences.
+struct PrefillCut {
+  int64_t items = 0;   // most workgroups of a grid of more than its row blocks (0: none is)
+  int64_t parts = 0;   // most of them in one that cuts spans: partials
+  int64_t blocks = 0;  // most row blocks of such a grid
+};
+inline PrefillCut prefill_cut(int64_t per_seq, int64_t batch, bool share, int units, int cus) {
+  PrefillCut c;
+  for (int64_t n = share ? 1 : batch; n <= batch && n * per_seq <= cus; ++n) {
+    const int split = prefill_split(units, n * per_seq, cus, share && n < batch);
+    if (split < 2) continue;
+    const int64_t items = n * per_seq * split;
+    c.items = c.items > items ? c.items : items;
+    if (prefill_split(units, n * per_seq, cus, false) < 2) continue;
+    c.parts = c.parts > items ? c.parts : items;
+    c.blocks = n * per_seq;
+  }
+  return c;
 }
 
 struct QuantRowsArgs {

@@ -186,7 +186,7 @@ __device__ __forceinline__ void zero_share(const Args &a, int64_t z, int64_t zen
 // The grid's work: live (sequence, KV head) segments, row blocks per segment and
 // pieces per span; `share`: a mixed batch, whose dead rows are shared out too.
 struct PrefillGrid {
-  int nseg, nblk, split;
+  int nseg, nblk, split;  // split: the most pieces of a span (prefill_split)
   bool share;
 };
 
@@ -206,7 +206,8 @@ __device__ __forceinline__ PrefillGrid prefill_grid(const AttnArgs &a, int lane)
     if (p.share) nseq = nlive;
   }
   p.nseg = nseq * a.g.hk;
-  p.split = a.pre_cus > 0 ? prefill_split((int64_t)p.nseg * p.nblk, a.pre_cus) : 1;
+  p.split = 1;
+  if (p.nseg * p.nblk <= a.pre_cus) p.split = prefill_split(a.pre_units, p.nseg * p.nblk, a.pre_cus, p.share);
   return p;
 }
 
@@ -231,19 +232,12 @@ __device__ __forceinline__ void prefill_item(const PrefillGrid &p, int bid, int 
     k = bid / p.nseg;
     seg = bid - k * p.nseg;
   }
-  piece = k % p.split;
-  rblk = p.nblk - 1 - k / p.split;
-}
-
-// Pieces a span of `stages` stages is cut into where the row blocks of the grid
-// are too few for the CUs (prefill_split): at least kSplitStages stages each (a
-// piece costs its start-up and 130 KB of partials, written and read).  One
-// sequence's chunk of 500 tokens behind 8,000 (64 row blocks, 4 pieces each)
-// 295 -> 98 us of kernel plus 14 us of merge; batches with a row block per CU
-// keep whole spans and no merge.
-constexpr int kSplitStages = 2;
-__device__ __forceinline__ int prefill_pieces(int stages, int split) {
-  return max(1, min(split, stages / kSplitStages));
+  piece = 0;
+  if (p.split > 1) {  // (no division for grids that cut nothing: 1.2 us of a two-round launch)
+    piece = k % p.split;
+    k /= p.split;
+  }
+  rblk = p.nblk - 1 - k;
 }
 
 template <int BITS, int DP, int G, int FK, bool SHARE>
@@ -274,7 +268,7 @@ __global__ __launch_bounds__(64 * kMaxPrefillWaves) void prefill_kernel(const At
   __shared__ __attribute__((aligned(16))) uint8_t s_valid[2][kStageTiles];
   __shared__ int s_lim[2][kPrefillWaves];
   __shared__ int64_t s_zero[SHARE ? 2 : 1];  // zero share: first row, end
-  __shared__ int s_item[3];  // pieces of the span, the block's piece, its partial
+  __shared__ int s_item[2];  // pieces of the span (0: none for this block), the block's partial
   __shared__ __attribute__((aligned(16))) uint16_t stage[2][I::ELEMS];
   // score metadata of the stage's K tiles (quantized pages)
   constexpr int SPG = BF16_BIAS ? 6 : bias_parts(NG);
@@ -390,14 +384,16 @@ __global__ __launch_bounds__(64 * kMaxPrefillWaves) void prefill_kernel(const At
   // start on page boundaries), so the stage loop holds no more than it does
   // for a whole span; what the epilogue needs of the item waits in LDS.
   if (pg.split > 1) {
-    constexpr int kAlign = kStageTiles < 8 ? 2 : 1;  // stages per 128 tokens (the largest page)
+    constexpr int kAlign = kPrefillUnit / (kStageTiles * PKV_TILE);  // stages per unit
     const int n = (nstages + kAlign - 1) / kAlign;
-    const int pieces = prefill_pieces(n, pg.split);
-    int s0 = 0, s1 = 0;
-    if (piece < pieces) {
-      s0 = n * piece / pieces * kAlign;
-      s1 = min(nstages, n * (piece + 1) / pieces * kAlign);
-    }
+    const int longest = prefill_longest((L - 1) / kPrefillUnit + 1, pg.nseg * nblk, a.pre_cus);
+    const int pieces = max(1, min((n + longest - 1) / longest, pg.split));
+    // a workgroup past the pieces has no stages, and at most a zero share to
+    // write (leaving here made the mixed batch's whole-span launch 1% slower; the
+    // grid has room for such workgroups beside the others: prefill_longest)
+    const bool none = piece >= pieces;
+    const int s0 = none ? 0 : n * piece / pieces * kAlign;
+    const int s1 = none ? 0 : min(nstages, n * (piece + 1) / pieces * kAlign);
     const int t0 = s0 * kStageTiles;
     ntiles = max(0, min(ntiles, s1 * kStageTiles) - t0);
     clear_tiles -= t0;
@@ -408,13 +404,11 @@ __global__ __launch_bounds__(64 * kMaxPrefillWaves) void prefill_kernel(const At
     for (int rb = 0; rb < RB; ++rb) lim[rb] -= lim[rb] < 0 ? 0 : t0 * PKV_TILE;  // < 0: nothing visible here
     if (tid == 0) {
       if (piece == 0) a.pre_cnt[seg * nblk + rblk] = pieces;
-      s_item[0] = pieces;
-      s_item[1] = piece;
-      s_item[2] = (seg * nblk + rblk) * pg.split + piece;
+      s_item[0] = none ? 0 : pieces;
+      s_item[1] = (seg * nblk + rblk) * pg.split + piece;
     }
   } else if (tid == 0) {
     s_item[0] = 1;
-    s_item[1] = 0;
   }
   const int tpp_shift = __builtin_ctz(g.page / PKV_TILE);
   const int tpp_mask = (1 << tpp_shift) - 1;
@@ -973,7 +967,6 @@ __global__ __launch_bounds__(64 * kMaxPrefillWaves) void prefill_kernel(const At
   LateArgs *late = (LateArgs *)__builtin_amdgcn_kernarg_segment_ptr();
   asm volatile("" : "+s"(late));
   const int pieces = __builtin_amdgcn_readfirstlane(s_item[0]);
-  const int piece_of = __builtin_amdgcn_readfirstlane(s_item[1]);
 #pragma unroll
   for (int rb = 0; rb < RB; ++rb) {
     if constexpr (MSUM) {
@@ -985,8 +978,7 @@ __global__ __launch_bounds__(64 * kMaxPrefillWaves) void prefill_kernel(const At
     if (pieces > 1) {
       // the piece's partial: (m, l) per row, O^T as the lanes hold it; rows
       // that are not live leave zeros
-      if (piece_of >= pieces) continue;
-      const int64_t blk = s_item[2];
+      const int64_t blk = s_item[1];
       const int rb16 = wv * RB + rb;
       const bool live = lim[rb] >= 0;
       if (jj == 0)
@@ -997,7 +989,7 @@ __global__ __launch_bounds__(64 * kMaxPrefillWaves) void prefill_kernel(const At
       continue;
     }
     const int row = rblk * ROWS + wv * 16 * RB + rb * 16 + col;
-    if (row >= late->rows || piece_of > 0) continue;
+    if (row >= late->rows || pieces == 0) continue;
     const int qi = row / late->gqa, h = kh * late->gqa + row % late->gqa;
     // dead rows (past the chunk's width) ran the unmasked steps: write 0
     const float inv = lim[rb] < 0 ? 0.0f : 1.0f / fmaxf(lsum[rb], 1e-20f);
@@ -1031,9 +1023,10 @@ __global__ __launch_bounds__(64 * kMaxPrefillWaves) void prefill_kernel(const At
 
 // ---- merge of split spans ----------------------------------------------------------
 
-// One wave per 16 rows of a row block whose span was cut: every piece's (m, l),
-// then the pieces' O^T in the lanes' own layout (1 KiB loads, a piece's NB of
-// them in flight together), weighted by 2^(m - M) and normalised.
+// One wave per 16 rows of a row block whose span was cut: every piece's (m, l)
+// and O^T in the lanes' own layout (1 KiB loads), weighted by 2^(m - M) and
+// normalised.  Bound by memory round trips, so several pieces are in flight
+// (four, two past head_dim 128), the first with the maxima.
 template <int DP, bool SHARE>
 __device__ __forceinline__ void prefill_merge(const AttnArgs &a, int unit) {
   constexpr int ROWS = prefill_rows(DP), RBLKS = ROWS / 16, NB = DP / 16;
@@ -1050,25 +1043,42 @@ __device__ __forceinline__ void prefill_merge(const AttnArgs &a, int unit) {
   if (b < 0 || b >= a.batch) return;
   const float *ml = a.pre_ml + ((int64_t)blk * pg.split * ROWS + rb16 * 16 + col) * 2;
   const float *src = a.pre_acc + ((int64_t)blk * pg.split * RBLKS + rb16) * (16 * DP) + lane * 4;
+  // pieces p0 .. p0 + FLY - 1, all requested at once
+  constexpr int FLY = DP > 128 ? 2 : 4;
+  float2 x[FLY];
+  f4 v[FLY][NB];
+  auto request = [&](int p0) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < FLY; ++i) {
+      const int p = min(p0 + i, pieces - 1);
+      x[i] = *(const float2 *)(ml + (int64_t)p * ROWS * 2);
+#pragma unroll
+      for (int n = 0; n < NB; ++n) v[i][n] = *(const f4 *)(src + (int64_t)p * RBLKS * (16 * DP) + n * 256);
+    }
+  };
+  request(0);
+  // the rows' maxima, the lanes of a row (jj) a quarter of the pieces each
   float M = -INFINITY;
-  for (int p = 0; p < pieces; ++p) {
-    const float2 x = *(const float2 *)(ml + (int64_t)p * ROWS * 2);
-    if (x.y != 0.0f) M = fmaxf(M, x.x);  // a piece without a visible token holds l = 0
+#pragma unroll 2
+  for (int p = jj; p < pieces; p += 4) {
+    const float2 y = *(const float2 *)(ml + (int64_t)p * ROWS * 2);
+    if (y.y != 0.0f) M = fmaxf(M, y.x);  // a piece without a visible token holds l = 0
   }
+  M = xor32_max(xor16_max(M));
   float L = 0.0f;
   f4 acc[NB];
 #pragma unroll
   for (int n = 0; n < NB; ++n) acc[n] = f4{0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll 2
-  for (int p = 0; p < pieces; ++p) {
-    const float2 x = *(const float2 *)(ml + (int64_t)p * ROWS * 2);
-    f4 v[NB];
+  for (int p0 = 0; p0 < pieces; p0 += FLY) {
+    if (p0 > 0) request(p0);
 #pragma unroll
-    for (int n = 0; n < NB; ++n) v[n] = *(const f4 *)(src + (int64_t)p * RBLKS * (16 * DP) + n * 256);
-    const float w = x.y != 0.0f ? __builtin_amdgcn_exp2f(x.x - M) : 0.0f;
-    L += w * x.y;
+    for (int i = 0; i < FLY; ++i) {
+      if (p0 + i >= pieces) break;
+      const float w = x[i].y != 0.0f ? __builtin_amdgcn_exp2f(x[i].x - M) : 0.0f;
+      L += w * x[i].y;
 #pragma unroll
-    for (int n = 0; n < NB; ++n) acc[n] += w * v[n];
+      for (int n = 0; n < NB; ++n) acc[n] += w * v[i][n];
+    }
   }
   if (row >= a.rows) return;
   const int qi = row / a.gqa, h = kh * a.gqa + row % a.gqa;
@@ -1150,13 +1160,8 @@ hipError_t launch_prefill(hipStream_t stream, const AttnArgs &a) {
     // device only: the grid covers any number of them; workgroups past the
     // pieces exit at once, but each needs a CU's LDS to start, so there are no
     // more than that)
-    const int64_t per_seq = blocks / a.batch;
-    int64_t most = share ? blocks : blocks * prefill_split(blocks, a.pre_cus);
-    for (int64_t n = per_seq; share && n <= blocks && n <= a.pre_cus; n += per_seq) {
-      const int64_t items = n * prefill_split(n, a.pre_cus);
-      most = items > most ? items : most;
-    }
-    blocks = most;
+    const int64_t items = prefill_cut(blocks / a.batch, a.batch, share, a.pre_units, a.pre_cus).items;
+    blocks = items > blocks ? items : blocks;
   }
   if (blocks > 0x7FFFFFFF) return hipErrorInvalidValue;
   hipLaunchKernelGGL(k, dim3((unsigned)blocks), dim3(64 * prefill_waves(a.g.dp)), 0, stream, a);
@@ -1176,9 +1181,8 @@ hipError_t launch_tail_merge(hipStream_t stream, const MergeArgs *tier, int tier
   t.pre = a;
   int64_t units = 0;
   if (prefill) {
-    // row blocks that can be split: those of a grid of at most pre_cus blocks
-    int64_t blocks = (int64_t)a.batch * a.g.hk * prefill_blocks(a.g, a.rows);
-    if (blocks > a.pre_cus) blocks = a.widths && a.narrow_q > 0 ? a.pre_cus : 0;
+    const int64_t blocks = prefill_cut((int64_t)a.g.hk * prefill_blocks(a.g, a.rows), a.batch,
+                                       a.widths && a.narrow_q > 0, a.pre_units, a.pre_cus).blocks;
     units = (blocks * (prefill_rows(a.g.dp) / 16) + nw - 1) / nw;
   }
   const int64_t grid = n[0] + n[1] + units;
