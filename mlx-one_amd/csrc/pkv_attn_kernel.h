@@ -481,8 +481,9 @@ __attribute__((amdgpu_waves_per_eu(min_waves_per_simd(BITS, DP, G, RB, SLOTS))))
   // codes and (scale, bias) words into the tile registers of the iteration
   // that holds it; no other wave reads that tile in this launch, so the
   // store needs no ordering against the tile loads.
-  __shared__ uint8_t s_app_codes[2][APPEND && QUANT ? DP : 4];
-  __shared__ uint16_t s_app_raw[2][APPEND && !QUANT ? DP : 2];  // float pages: the rows themselves
+  // (read by words in patch_k)
+  __shared__ __attribute__((aligned(16))) uint8_t s_app_codes[2][APPEND && QUANT ? DP : 4];
+  __shared__ __attribute__((aligned(16))) uint16_t s_app_raw[2][APPEND && !QUANT ? DP : 2];  // float pages: the rows
   __shared__ uint32_t s_app_meta[2][8];
   int app_it = -1, app_j = 0, app_tt = 0;
   // the new rows are requested with the piece's queries, ahead of its tiles
