@@ -111,10 +111,11 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void va
   }
   const int t0 = __builtin_amdgcn_readfirstlane(all_tiles) * hk;
   if (t0 == 0) return;
-  lead = charged_lead(a.seq_lens, a.widths, a.narrow_lo, a.narrow_q, a.batch, a.waves, a.lead, nt_l, t0, lane);
+  lead = charged_lead(a.seq_lens, a.widths, a.narrow_lo, a.narrow_q, a.batch, a.waves, a.least, a.lead, nt_l, t0,
+                      lane);
   scan_chunk(0, 0);
   const int T = t0 + __builtin_amdgcn_readfirstlane(served) * hk * lead;
-  const int W = min(a.waves, T);
+  const int W = split_runs(a.waves, a.least, T);
   if (w >= W) return;
   Split sp;
   sp.init(T, W);

@@ -177,10 +177,11 @@ __attribute__((amdgpu_waves_per_eu(min_waves_per_simd(BITS, DP, G, RB, SLOTS))))
     // tile counts fit in int32: the host bounds batch * (max_pages * pages' tiles + 16) * HK
     const int t0 = __builtin_amdgcn_readfirstlane(all_tiles) * hk;
     if (t0 == 0) return;  // every sequence is served by the prefill kernel
-    lead = charged_lead(a.seq_lens, a.widths, a.narrow_lo, a.narrow_q, a.batch, a.waves, a.lead, nt_l, t0, lane);
+    lead = charged_lead(a.seq_lens, a.widths, a.narrow_lo, a.narrow_q, a.batch, a.waves, a.least, a.lead, nt_l, t0,
+                        lane);
     scan_chunk(0, 0);
     const int T = t0 + __builtin_amdgcn_readfirstlane(served) * hk * lead;
-    const int W = min(a.waves, T);
+    const int W = split_runs(a.waves, a.least, T);
     if (w >= W) return;
     sp.init(T, W);
   }

@@ -54,6 +54,7 @@ struct AttnArgs {
   // otherwise runs one wave per run (else 0), and whether run w is segment w,
   // whole, instead of an equal share of the tiles (no partials, no merge).
   int group = 0, seg_runs = 0;
+  int least = 0;     // a run holds 2^least tiles at least (fewer runs where there are too few tiles)
   int lead;          // tiles of start-up cost charged ahead of each segment in the split
   float *part_acc;   // [2*waves][rows][DP]
   float *part_ml;    // [2*waves][rows][2]
@@ -74,7 +75,7 @@ struct AttnArgs {
 
 struct MergeArgs {
   int batch, hk, heads, nq, gqa, rows, dim, dp, float_kind;
-  int waves, lead;  // as launched for the attention kernel
+  int waves, lead, least = 0;  // as launched for the attention kernel
   int nq_stride, narrow_lo, narrow_q;
   const int32_t *seq_lens, *widths;
   const float *part_acc, *part_ml;

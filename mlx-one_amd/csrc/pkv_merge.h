@@ -60,16 +60,21 @@ __device__ __forceinline__ int split_tiles(const int32_t *lens, const int32_t *w
   return seq_tiles(lens[idx]);
 }
 
+// Runs of a launch over T split tiles: `runs`, or as few as leave each 2^least tiles.
+__device__ __forceinline__ int split_runs(int runs, int least, int T) {
+  return min(runs, ((T - 1) >> least) + 1);
+}
+
 // The lead tiles a launch's split charges ahead of each segment: `lead`, or
 // none when the lead-free split's equal runs already end on segment
 // boundaries (every sequence's tile count a multiple of the run length), so
 // that no run crosses one.  nt0: the lane's tile count in the first
 // 64-sequence chunk; t0: the lead-free tile total over all segments.
 __device__ __forceinline__ int charged_lead(const int32_t *lens, const int32_t *widths, int narrow_lo,
-                                            int narrow_q, int batch, int waves, int lead, int nt0,
+                                            int narrow_q, int batch, int waves, int least, int lead, int nt0,
                                             int t0, int lane) {
   if (lead == 0 || t0 == 0) return 0;
-  const int w0 = min(waves, t0);
+  const int w0 = split_runs(waves, least, t0);
   if (t0 % w0) return lead;
   const int q0 = t0 / w0;
   bool off = lane < batch && nt0 % q0 != 0;
@@ -114,13 +119,13 @@ __device__ __forceinline__ void merge_unit(const MergeArgs &a, int unit) {
   }
   const int ntb = split_tiles(a.seq_lens, a.widths, a.narrow_lo, a.narrow_q, b);
   const int t0 = __builtin_amdgcn_readfirstlane(tiles) * a.hk;
-  const int lead = charged_lead(a.seq_lens, a.widths, a.narrow_lo, a.narrow_q, a.batch, a.waves, a.lead, nt0,
+  const int lead = charged_lead(a.seq_lens, a.widths, a.narrow_lo, a.narrow_q, a.batch, a.waves, a.least, a.lead, nt0,
                                 t0, lane);
   const int T = t0 + __builtin_amdgcn_readfirstlane(served) * a.hk * lead;
   const int sv = (__builtin_amdgcn_readfirstlane(pre) + __builtin_amdgcn_readfirstlane(spre) * lead) *
                      a.hk + kh * (ntb + lead);
   Split sp;
-  sp.init(T, min(a.waves, T));
+  sp.init(T, split_runs(a.waves, a.least, T));
   const SegPieces pc = seg_pieces(sp, sv, sv + lead, sv + lead + ntb);
   if (pc.n < 2) return;  // the same for every wave of the workgroup
 
