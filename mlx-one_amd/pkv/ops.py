@@ -229,12 +229,16 @@ def attention_workspace(device, nbytes):
     return ws
 
 
-def _wide_workspace(device, nbytes):
+def _wide_workspace(device, nbytes, least):
     """The workspace of a wide call that was given none: the stream's own memory
     of exactly that size -- wide calls on other streams or threads may overlap
     it, and whether spans are cut (and so the output's bits) must not depend on
-    what grew the shared one."""
-    return torch.empty(max(nbytes, 256), dtype=torch.uint8, device=device)
+    what grew the shared one.  Without room for it, ``least()`` bytes, with
+    which the call runs whole spans."""
+    try:
+        return torch.empty(max(nbytes, 256), dtype=torch.uint8, device=device)
+    except torch.OutOfMemoryError:
+        return torch.empty(max(least(), 256), dtype=torch.uint8, device=device)
 
 
 def paged_attention(fmt: PageFormat, pool, queries, block_table, seq_lens, *, scale, q_pos=None,
@@ -267,7 +271,8 @@ def paged_attention(fmt: PageFormat, pool, queries, block_table, seq_lens, *, sc
     else:
         need, wide = call_workspace_bytes(fmt, heads, nq, batch, waves), is_wide(fmt, heads, nq)
     if workspace is None:
-        workspace = _wide_workspace(device, need) if wide else attention_workspace(device, need)
+        workspace = (_wide_workspace(device, need, lambda: workspace_bytes(fmt, heads, nq, waves))
+                     if wide else attention_workspace(device, need))
     elif workspace.device != device or workspace.dtype != torch.uint8 or \
             not workspace.is_contiguous():
         raise ValueError("attention workspace must be a contiguous uint8 tensor on the "
@@ -315,7 +320,8 @@ def append_paged_attention(fmt: PageFormat, pool, keys, values, queries, block_t
     else:
         need, wide = call_workspace_bytes(fmt, heads, 1, batch, waves), is_wide(fmt, heads, 1)
     if workspace is None:
-        workspace = _wide_workspace(device, need) if wide else attention_workspace(device, need)
+        workspace = (_wide_workspace(device, need, lambda: 0) if wide
+                     else attention_workspace(device, need))
     elif workspace.device != device or workspace.dtype != torch.uint8 or \
             not workspace.is_contiguous():
         raise ValueError("attention workspace must be a contiguous uint8 tensor on the "

@@ -105,3 +105,43 @@ def test_captured_step_equals_the_eager_one():
         arena.truncate(slots, before)
         eager = runner.execute(slots, step.hidden)
         assert torch.equal(out, eager)
+
+
+def test_without_room_for_partials_the_call_runs_whole_spans(monkeypatch):
+    """The partials' memory refused (a full device): the wide call and the wide
+    step take the small workspace and give whole spans' bits."""
+    from pkv import ops
+
+    gen = torch.Generator(device="cuda").manual_seed(2)
+    fmt = ops.PageFormat(2, 64, 16, 8, 64)
+    n, nq = 2000, 70
+    per = -(-n // 16)
+    table = torch.randperm(2 * per, generator=gen, device="cuda").to(torch.int32).view(2, per)
+    pool = ops.allocate_pool(fmt, 2 * per)
+    lens = torch.tensor([n, 1200], dtype=torch.int32, device="cuda")
+    widths = torch.tensor([nq, 1], dtype=torch.int32, device="cuda")
+    k, v = (torch.randn((2, 2, n, 64), generator=gen, device="cuda").to(fmt.dtype) for _ in range(2))
+    ops.append_quantize(fmt, pool, k, v, table, torch.zeros_like(lens), lens)
+    q = torch.randn((2, 8, nq, 64), generator=gen, device="cuda").to(fmt.dtype)
+    waves = ops.split_waves(fmt, 8, nq, 2, q.device)
+    small = torch.empty(ops.workspace_bytes(fmt, 8, nq, waves), dtype=torch.uint8, device="cuda")
+    call = lambda **kw: ops.paged_attention(fmt, pool, q, table, lens, scale=0.125, widths=widths, **kw)
+    whole = call(waves=waves, workspace=small)
+    step, _ = _case(40)
+    empty, refused, limit = torch.empty, [], [small.numel()]
+
+    def full(*args, **kw):
+        if kw.get("dtype") is torch.uint8 and args[0] > limit[0]:
+            refused.append(args[0])
+            raise torch.OutOfMemoryError
+        return empty(*args, **kw)
+
+    cut = step()
+    monkeypatch.setattr(torch, "empty", full)
+    assert torch.equal(call(), whole) and len(refused) == 1
+    limit[0] = 256
+    out = step()
+    monkeypatch.undo()
+    assert len(refused) == 2 and torch.isfinite(out).all()
+    bound = cut.float().abs() * 2.0 ** -7 + cut.float().abs().amax(-1, keepdim=True) * 2.0 ** -8 + 1e-6
+    assert bool(((out.float() - cut.float()).abs() <= bound).all())
