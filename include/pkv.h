@@ -142,11 +142,13 @@ int pkv_paged_attention(void *stream, const pkv_layout *layout, const void *pool
  * attend its one query (as pkv_paged_attention with num_queries = 1, q_pos
  * NULL, widths NULL), in one launch where the decode kernel serves the shape
  * (at most 8 query rows per KV head): the wave that attends a sequence's last
- * tile quantizes the new token, stores it and uses it.
+ * tile quantizes the new token (float pages: copies it), stores it and uses it.
  * Other shapes run the append and the attention as two launches.  Replaces
  * the append-then-attend pair of PagedBatchCache.attend (engine/paged.py:
- * 260-263) for a decode step; pages and output equal the two separate calls'
- * bit for bit.
+ * 260-263) for a decode step.  Pages equal the two separate calls' bit for bit
+ * (both drop a token past the block table); the output agrees to the rounding
+ * of another split, two steps of its 16-bit type plus 2^-8 of the row's largest
+ * element.
  *
  *  pool         : writable (the new tokens land in it)
  *  keys, values : [batch][HK][1][head_dim], float_kind

@@ -340,15 +340,16 @@ int paged_attention_impl(void *stream, const pkv_layout *layout, const void *poo
   // rows per KV head (the 4-row column-slot kernel) and the wider ones up to
   // the kernel's limit, so decode rows do not run at verify cost -- when the
   // workspace holds each tier's partials (else the prefill kernel serves
-  // every sequence).  The tiers run one after the other on the stream and
-  // share the workspace.
+  // every sequence).  The tiers run one after the other on the stream;
+  // with room for it each has a region of the workspace and one launch merges
+  // them, else they share one and each is merged before the next.
   struct Part {
     int nq, lo, hi, waves;  // queries covered; serve widths in (lo, hi] (hi 0: all)
     WorkspaceParts ws;
   };
   Part part[2];
   // the decode kernel appends the single new token itself (else an append
-  // launch goes first): the fused form runs one wave per run
+  // launch goes first), in the run form the shape has without it
   const int in_kernel_append = fused && !wide && pkv::append_fusable(pkv::to_geo(geo), rows) ? 1 : 0;
   int nparts = 0;
   if (!wide) {

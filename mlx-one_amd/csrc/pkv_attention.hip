@@ -581,7 +581,7 @@ static AttnKernel select_valu(const Geo &g) {
 
 // Rows per KV head -> column slots: <= 4 rows: 4 slots, <= 8: 2, else 1
 // (two row blocks past 16 rows).  With the fused single-token append: the
-// MFMA kernels of up to 8 rows over quantized pages (else none).
+// MFMA kernels of up to 8 rows (else none).
 static AttnKernel select_kernel(const Geo &g, int rows, bool append = false) {
   if (append) {
     if (rows <= 4) return select_shape<1, 4, true, false>(g);

@@ -95,8 +95,6 @@ __device__ __forceinline__ void lds_barrier() {
   asm volatile("s_barrier" ::: "memory");
 }
 
-// Query rows of sequence b live in this launch: 0 for a sequence of a mixed
-// batch that the decode kernel serves (narrow_q > 0, width at most narrow_q).
 // f32 -> bf16 bits on v_cvt_pk_bf16_f32 (round to nearest even): for the
 // values an f16 holds (never f32 denormals) the bits of f32_to_bf16_bits,
 // without its software NaN branch.
@@ -104,6 +102,8 @@ __device__ __forceinline__ uint16_t bf16_bits_cvt(float x) {
   return __builtin_bit_cast(uint16_t, (__bf16)x);
 }
 
+// Query rows of sequence b live in this launch: 0 for a sequence of a mixed
+// batch that the decode kernel serves (narrow_q > 0, width at most narrow_q).
 template <typename Args>
 __device__ __forceinline__ int prefill_width(const Args &a, int b) {
   return a.widths ? (a.narrow_q > 0 && a.widths[b] <= a.narrow_q ? 0 : a.widths[b]) : a.nq;

@@ -1,8 +1,8 @@
 """GPU: the fused single-token step (``pkv_append_paged_attention``) through the C ABI.
 
 One launch appends each sequence's new K/V token and attends its query where
-the decode kernel serves the shape (quantized pages, <= 8 query rows per KV
-head); other shapes run an append launch and the attention.  Either way the
+the decode kernel serves the shape (<= 8 query rows per KV head); other
+shapes run an append launch and the attention.  Either way the
 pages must equal ``pkv_append_quantize`` followed by ``pkv_paged_attention``
 bit for bit, and both outputs must meet the oracle's bar
 (``engine/paged.py:260-263`` is the reference's append-then-attend pair).
@@ -88,7 +88,7 @@ CASES = {
     "int4_d256_g64_p32": (dict(name="c3", batch=2, lengths=(200, 45), head_dim=256), 0),
     "int8_g128_gqa8_p64": (dict(name="c2", batch=4, lengths=(64, 65, 500, 3), kv_heads=4,
                                 group_size=128, page_tokens=64), 0),
-    # served by two launches inside the entry point
+    # float pages (the rows stored as they are), and a shape served by two launches
     "fallback_bf16_pages": (dict(name="c2", batch=3, lengths=(40, 3, 70), bits=16,
                                  group_size=32), 0),
     "fallback_rows16": (dict(name="c2", batch=3, lengths=(50, 18, 200), heads=32, kv_heads=2), 0),
